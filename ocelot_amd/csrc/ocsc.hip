@@ -145,12 +145,12 @@ __global__ void k_setup(KickScalars* __restrict__ s, KickInputs in) {
 // gridDim.x workgroups (k_fold), and the last workgroup to finish runs this
 // kick's set-up and the frame reduction (k_setup, k_reduceA): one launch
 // instead of three.  The same sums bit for bit: each workgroup folds the same
-// chunk, and reducing the gridDim.x (<= 256) folded values with 256 threads
-// takes the tree that 1024 threads would (the extra lanes add only zeros).
+// chunk, and the reduction of the gridDim.x folded values takes one wavefront
+// per component whatever the workgroup's size.
 __global__ void __launch_bounds__(256) k_fold_frame(const double* __restrict__ part, int nblk,
                                                     double* __restrict__ folded, KickScalars* __restrict__ sc,
                                                     KickInputs in) {
-  __shared__ double lds[16 * 3];
+  __shared__ double lds[4 * 3];
   __shared__ int last;
   const int nf = gridDim.x, chunk = (nblk + nf - 1) / nf;
   const int b0 = blockIdx.x * chunk, b1 = b0 + chunk < nblk ? b0 + chunk : nblk;
@@ -682,11 +682,16 @@ KickInputs kick_inputs(const int32_t* nmesh, int64_t n, double E_GeV, double zst
 // grid of the strided reduction passes (A, B, moments): one full round of
 // resident workgroups (no tail of half-empty rounds), at most one per 8 * 256
 // particles (every thread sums several particles before the workgroup's
-// reduction tree, which costs more than one particle's transform: batched
-// passes over bunches of a few 1e5 particles ran at half the bandwidth)
+// reduction tree: the passes over a batch's bunches of a few 1e5 particles
+// take 268 us at 8 particles per thread, 305 at 2) unless that leaves CUs
+// without a workgroup: then one per CU, down to one particle per thread
+// (20k particles: pass A 9.2 -> 3.8 us, pass B 12.1 -> 5.5 us; 333k: 10.6 ->
+// 8.0 and 13.0 -> 10.7 us)
 constexpr int64_t kRedParticles = 8 * kPT;
+constexpr int64_t kRedMinBlocks = 256;  // one workgroup per CU
 int nred_blocks(const ocsc_ctx* c, int64_t n) {
-  int64_t b = (n + kRedParticles - 1) / kRedParticles;
+  const int64_t full = (n + kRedParticles - 1) / kRedParticles, most = (n + kPT - 1) / kPT;
+  const int64_t b = std::max(full, std::min(most, kRedMinBlocks));
   return (int)(b < c->red_blocks ? (b < 1 ? 1 : b) : c->red_blocks);
 }
 

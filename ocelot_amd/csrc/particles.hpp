@@ -142,9 +142,15 @@ __device__ __forceinline__ void grid_coords(const double* xyz, const KickScalars
 }
 
 // ---------------------------------------------------------------------------
-// Deterministic block reductions: wave shuffles, then the waves' results in
-// a fixed order.  KIND 0: every value is a sum; KIND 1 (pass B layout):
-// values 0-2 minima, 3-5 maxima, the rest sums.
+// Deterministic block reductions in a fixed order.  KIND 0: every value is a
+// sum; KIND 1 (pass B layout): values 0-2 minima, 3-5 maxima, the rest sums.
+//
+// What bounds them is latency: the trees sit at the end of every particle
+// pass and make up the single-workgroup kernels between the passes.  Inside a
+// wavefront values move by DPP (row shifts, then row broadcasts): a step is
+// two 4-cycle register moves per double where a shuffle is two trips through
+// the LDS pipe.  Measured (MI355X): the 11-value reduction kernel of a kick
+// 9.3 -> 3.3 us at 10 partials; see reduce_partials for the larger counts.
 template <int KIND>
 __device__ __forceinline__ double red_op(int c, double a, double b) {
   if (KIND == 1 && c < 3) return b < a ? b : a;
@@ -152,60 +158,95 @@ __device__ __forceinline__ double red_op(int c, double a, double b) {
   return a + b;
 }
 
-// result valid in thread 0; lds holds (blockDim/64) * NV doubles
+template <int KIND>
+__device__ __forceinline__ double red_id(int c) {
+  if (KIND == 1 && c < 3) return __builtin_inf();
+  if (KIND == 1 && c < 6) return -__builtin_inf();
+  return 0.0;
+}
+
+// v of the lane that the DPP control CTRL reads from, `old` where it names
+// none (or the row is masked out)
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_from(double v, double old) {
+  const int2 s = __builtin_bit_cast(int2, v), o = __builtin_bit_cast(int2, old);
+  const int2 r = {__builtin_amdgcn_update_dpp(o.x, s.x, CTRL, ROWS, 0xf, false),
+                  __builtin_amdgcn_update_dpp(o.y, s.y, CTRL, ROWS, 0xf, false)};
+  return __builtin_bit_cast(double, r);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const int2 s = __builtin_bit_cast(int2, v);
+  const int2 r = {__builtin_amdgcn_readlane(s.x, lane), __builtin_amdgcn_readlane(s.y, lane)};
+  return __builtin_bit_cast(double, r);
+}
+
+// NV values reduced over the 64 lanes of a wavefront (all of them active);
+// the results are uniform.  c0: the component of v[0] (KIND 1)
+template <int NV, int KIND>
+__device__ __forceinline__ void wave_reduce(double* v, int c0 = 0) {
+#define OCSC_RED_STEP(CTRL, ROWS)                                                                          \
+  _Pragma("unroll") for (int c = 0; c < NV; ++c) v[c] =                                                    \
+      red_op<KIND>(c0 + c, v[c], dpp_from<CTRL, ROWS>(v[c], red_id<KIND>(c0 + c)))
+  OCSC_RED_STEP(0x111, 0xf);  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row
+  OCSC_RED_STEP(0x112, 0xf);
+  OCSC_RED_STEP(0x114, 0xf);
+  OCSC_RED_STEP(0x118, 0xf);
+  OCSC_RED_STEP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  OCSC_RED_STEP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3: lane 63 holds the wavefront
+#undef OCSC_RED_STEP
+#pragma unroll
+  for (int c = 0; c < NV; ++c) v[c] = lane_value(v[c], 63);
+}
+
+// result valid in the first wavefront; lds holds (blockDim/64) * NV doubles
 template <int NV, int KIND>
 __device__ __forceinline__ void block_reduce(double* v, double* lds) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int c = 0; c < NV; ++c) v[c] = red_op<KIND>(c, v[c], __shfl_down(v[c], off, 64));
+  static_assert(NV <= 64, "one lane per value");
+  wave_reduce<NV, KIND>(v);
   const int w = threadIdx.x >> 6, nw = blockDim.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0)
 #pragma unroll
     for (int c = 0; c < NV; ++c) lds[w * NV + c] = v[c];
   __syncthreads();
-  // the waves' results combined by the same shuffle tree in wave 0
+  // lane c adds the wavefronts' values of component c in order
   if (w == 0) {
+    const int c0 = lane < NV ? lane : 0;
+    double t = lds[c0];
+    for (int k = 1; k < nw; ++k) t = red_op<KIND>(c0, t, lds[k * NV + c0]);
 #pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      const double id = (KIND == 1 && c < 3) ? __builtin_inf() : ((KIND == 1 && c < 6) ? -__builtin_inf() : 0.0);
-      v[c] = lane < nw ? lds[lane * NV + c] : id;
-    }
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1)
-#pragma unroll
-      for (int c = 0; c < NV; ++c) v[c] = red_op<KIND>(c, v[c], __shfl_down(v[c], off, 64));
+    for (int c = 0; c < NV; ++c) v[c] = lane_value(t, c);
   }
 }
 
-// partials are stored transposed, part[c * nblk + b], so the final reduction
-// reads them coalesced
+// Totals of nblk partials of NV components, stored transposed (part[c * nblk
+// + b], coalesced): a wavefront takes whole components, its lanes adding
+// every 64th partial (U loads in flight, added in increasing b), so a
+// component needs one wavefront reduction instead of one per wavefront of the
+// workgroup.  out is valid in every thread; lds holds NV doubles.  The 11
+// components of 977 partials: 10.7 -> 5.2 us, 12 of 2048: 10.0 -> 5.0 us (a
+// workgroup of 16 wavefronts, each reducing every component by shuffles,
+// before).
 template <int NV, int KIND>
 __device__ __forceinline__ void reduce_partials(const double* __restrict__ part, int nblk, double* out, double* lds) {
-  double v[NV];
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  constexpr int U = 8;
+  for (int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); c < NV; c += nw) {
+    double v = red_id<KIND>(c);
+    const double* p = part + (int64_t)c * nblk;
+    for (int b0 = lane; b0 < nblk; b0 += U * 64) {
+      double t[U];
 #pragma unroll
-  for (int c = 0; c < NV; ++c) v[c] = KIND == 1 && c < 3 ? __builtin_inf() : (KIND == 1 && c < 6 ? -__builtin_inf() : 0.0);
-  // U partials per thread are loaded before any is combined, so U loads are
-  // in flight instead of one; each thread still combines its partials in
-  // increasing b (out-of-range slots are skipped), so the tree is unchanged
-  constexpr int U = NV > 8 ? 2 : (NV > 4 ? 4 : 8);
-  for (int b0 = threadIdx.x; b0 < nblk; b0 += U * blockDim.x) {
-    double t[U][NV];
+      for (int u = 0; u < U; ++u) t[u] = b0 + u * 64 < nblk ? p[b0 + u * 64] : red_id<KIND>(c);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int b = b0 + u * blockDim.x;
-#pragma unroll
-      for (int c = 0; c < NV; ++c) t[u][c] = b < nblk ? part[c * nblk + b] : 0.0;
+      for (int u = 0; u < U; ++u) v = red_op<KIND>(c, v, t[u]);
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (b0 + u * (int)blockDim.x < nblk)
-#pragma unroll
-        for (int c = 0; c < NV; ++c) v[c] = red_op<KIND>(c, v[c], t[u][c]);
+    wave_reduce<1, KIND>(&v, c);
+    if (lane == 0) lds[c] = v;
   }
-  block_reduce<NV, KIND>(v, lds);
+  __syncthreads();
 #pragma unroll
-  for (int c = 0; c < NV; ++c) out[c] = v[c];
+  for (int c = 0; c < NV; ++c) out[c] = lds[c];
 }
 
 // First level of a two-level sum over many block partials: block f of the
@@ -281,7 +322,7 @@ __global__ void __launch_bounds__(kPT) k_passA(Rows R, KickScalars* __restrict__
 // frame from the mean momentum (sc.py:224-239)
 __device__ __forceinline__ void reduceA_body(KickScalars* __restrict__ scp, const double* __restrict__ part, int nblk,
                                              const int bx, const int nbx) {
-  __shared__ double lds[16 * 3];
+  __shared__ double lds[3];
   double acc[3];
   reduce_partials<3, 0>(part, nblk, acc, lds);
   if (threadIdx.x != 0) return;
@@ -394,51 +435,54 @@ __global__ void __launch_bounds__(kPT) k_passB(Rows R, const double* __restrict_
 // (sc.py:172-186)
 __device__ __forceinline__ void reduceB_body(KickScalars* __restrict__ scp, const double* __restrict__ part, int nblk,
                                              int prec, const int bx, const int nbx) {
-  __shared__ double lds[16 * kNPartB];
+  __shared__ double tot[kNPartB];
   double out[kNPartB];
-  reduce_partials<kNPartB, 1>(part, nblk, out, lds);
-  const int tid = threadIdx.x;
-  if (tid != 0) return;
+  reduce_partials<kNPartB, 1>(part, nblk, out, tot);
+  if (threadIdx.x >= 64) return;
+  // lanes 0-2 take an axis each (its five divisions are one dependent chain)
   KickScalars& s = *scp;
-  int err = s.err;
-  for (int k = 0; k < 3; ++k) {
-    s.xmin[k] = out[k];
-    s.xmax[k] = out[3 + k];
-    s.sumqx[k] = out[8 + k];
-  }
-  s.sumq = out[6];
-  s.sumabsq = out[7];
-  bool same = s.key_prec == prec;
-  for (int k = 0; k < 3; ++k) {
-    double XX = s.xmax[k] - s.xmin[k];
+  const double sumq = out[6];
+  const int k = threadIdx.x;
+  int e = 0;
+  bool same = true;
+  double h = 0;
+  if (k < 3) {
+    const double xmin = tot[k], xmax = tot[3 + k], sumqx = tot[8 + k];
+    s.xmin[k] = xmin;
+    s.xmax[k] = xmax;
+    s.sumqx[k] = sumqx;
+    double XX = xmax - xmin;
     if (s.random_mesh) XX = XX * s.mesh_scale;
-    const double h = XX / (double)(s.nmesh[k] - 3);
+    h = XX / (double)(s.nmesh[k] - 3);
     s.steps[k] = h;
     s.inv_steps[k] = 1.0 / h;
-    if (!(h > 0) || !__builtin_isfinite(h)) err |= kErrSteps;
-    const double Xmin = s.xmin[k] / h;
-    const double Xmid = (s.sumqx[k] / h) / s.sumq;
+    if (!(h > 0) || !__builtin_isfinite(h)) e |= kErrSteps;
+    const double Xmin = xmin / h;
+    const double Xmid = (sumqx / h) / sumq;
     double off = __builtin_floor(Xmin - Xmid) + Xmid;
     if (s.random_mesh) off = off + s.mesh_shift;
     s.X_off[k] = off;
-    if (!__builtin_isfinite(off)) err |= kErrZeroCharge;
-    same = same && s.key_steps[k] == h && s.key_nmesh[k] == s.nmesh[k];
+    if (!__builtin_isfinite(off)) e |= kErrZeroCharge;
+    same = s.key_steps[k] == h && s.key_nmesh[k] == s.nmesh[k];
   }
-  if (s.sumq == 0) err |= kErrZeroCharge;
+  same = __ballot(!same) == 0 && s.key_prec == prec;
+  int err = s.err;
+  if (__ballot(e & kErrSteps)) err |= kErrSteps;
+  if (__ballot(e & kErrZeroCharge) || sumq == 0) err |= kErrZeroCharge;
+  if (!same && k < 3) {
+    s.key_steps[k] = h;
+    s.key_nmesh[k] = s.nmesh[k];
+  }
+  if (k != 0) return;
+  s.sumq = sumq;
+  s.sumabsq = out[7];
   int e2 = 0;
   const double fr = __builtin_frexp(s.sumabsq, &e2);
   (void)fr;
   s.qscale = __builtin_ldexp(1.0, 62 - e2);
   s.inv_qscale = __builtin_ldexp(1.0, e2 - 62);
-  s.rebuild = same ? 0 : 1;
-  if (!same) {
-    for (int k = 0; k < 3; ++k) {
-      s.key_steps[k] = s.steps[k];
-      s.key_nmesh[k] = s.nmesh[k];
-    }
-    s.key_prec = prec;
-  }
-  if (err) s.rebuild = 1;
+  if (!same) s.key_prec = prec;
+  s.rebuild = same && !err ? 0 : 1;
   s.err = err;
 }
 
