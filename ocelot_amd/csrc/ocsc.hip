@@ -145,8 +145,8 @@ __global__ void k_setup(KickScalars* __restrict__ s, KickInputs in) {
 // gridDim.x workgroups (k_fold), and the last workgroup to finish runs this
 // kick's set-up and the frame reduction (k_setup, k_reduceA): one launch
 // instead of three.  The same sums bit for bit: each workgroup folds the same
-// chunk, and the reduction of the gridDim.x folded values takes one wavefront
-// per component whatever the workgroup's size.
+// chunk, and reducing the gridDim.x (<= 256) folded values with 256 threads
+// takes the tree that 1024 threads would (the extra lanes add only zeros).
 __global__ void __launch_bounds__(256) k_fold_frame(const double* __restrict__ part, int nblk,
                                                     double* __restrict__ folded, KickScalars* __restrict__ sc,
                                                     KickInputs in) {
@@ -694,6 +694,15 @@ int nred_blocks(const ocsc_ctx* c, int64_t n) {
   const int64_t b = std::max(full, std::min(most, kRedMinBlocks));
   return (int)(b < c->red_blocks ? (b < 1 ? 1 : b) : c->red_blocks);
 }
+// The frame and extent passes: the mixed form keeps 8 particles per thread at
+// every size.  Another split moves the frame in its last bits and with it the
+// FP32 rounding of every field value (1e-7 of the kick, where the FP64 form
+// moves 1e-15).
+int frame_blocks(const ocsc_ctx* c, int64_t n, int prec) {
+  if (prec == OCSC_FP64) return nred_blocks(c, n);
+  const int64_t b = (n + kRedParticles - 1) / kRedParticles;
+  return (int)(b < c->red_blocks ? (b < 1 ? 1 : b) : c->red_blocks);
+}
 
 // read back one timed kick of the profiling ring
 int flush_slot(ocsc_ctx* c, int k) {
@@ -805,7 +814,7 @@ template <typename F, int NWORD>
 int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld, const double* q, const KickInputs& in,
                  int prec, hipStream_t st, const StepOpts& o = StepOpts()) {
   const int64_t n = in.n;
-  const int nblk = nred_blocks(c, n);
+  const int nblk = frame_blocks(c, n, prec);
   const int npart = (int)((n + kKickPT - 1) / kKickPT);  // kick workgroups
   Rows R{r, ld};
   const bool prof = c->profiling != 0;
@@ -1502,7 +1511,7 @@ int ocsc_el_field(ocsc_ctx* c, const double* xyz, int64_t ld, const double* q, i
   } xcd_off{c, c->deposit_xcd};
   c->deposit_xcd = 0;
   in.gamma0 = gamma;
-  const int nblk = nred_blocks(c, n);
+  const int nblk = frame_blocks(c, n, prec);
   const int npart = (int)((n + kPT - 1) / kPT);
   Rows R{xyz, ld};
   k_setup<<<1, 64, 0, st>>>(L.sc, in);
@@ -1873,10 +1882,11 @@ LscConst lsc_const(int step_profile, double smooth, double E_GeV, double dz, dou
                    int cap);
 constexpr int kLscGraphBins = 4096;  // kicks inside tracking graphs (device-planned grid; 32 KB of LDS)
 // the LSC kick's momentum sums for the next space-charge kick (the pass-A
-// partials of the kick scalars sc, nred_blocks of them)
+// partials of the kick scalars sc, nblk of them)
 struct LscSump {
   const KickScalars* sc;
   double* part;
+  int nblk;
 };
 int enqueue_lsc(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, const LscConst& k, double b0,
                 double b1, hipStream_t st, const DriftArgs* dr = nullptr, const LscSump* sm = nullptr);
@@ -2058,7 +2068,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
       // drift here; the LSC kick leaves the next kick's momentum sums, in
       // pass A's partial layout
       o.drift = o.sump = false;
-      o.prev_nblk = nred_blocks(c, n);
+      o.prev_nblk = frame_blocks(c, n, prec);
     }
     o.dr = DriftArgs{Ld, r56};
     o.grid_zeroed = c->grid_clear == 2 && step > 0;
@@ -2088,7 +2098,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
     // the next drift: fused into the LSC kick when there are no moments
     const DriftArgs next{Ld, r56};
     const bool fuse = lq && !tw && step < nsteps - 1;
-    const LscSump sm{L.sc, (double*)L.part.p};  // read by the next step's kick
+    const LscSump sm{L.sc, (double*)L.part.p, frame_blocks(c, n, prec)};  // read by the next step's kick
     if (lq && (rc3 = enqueue_lsc(c, rr, lr, qq, n, lq->k, lq->b0, lq->b1, s2, fuse ? &next : nullptr,
                                  step < nsteps - 1 ? &sm : nullptr)))
       return rc3;
@@ -2344,7 +2354,7 @@ int fused_plan(ocsc_ctx* c, const std::vector<int>& kicked, const std::vector<do
     b.n = nn[i];
     b.sc = L.sc;
     b.part = (double*)L.part.p;
-    b.nblk = nred_blocks(c, nn[i]);
+    b.nblk = frame_blocks(c, nn[i], prec);
     b.d = g.d;
     b.ncell = g.ncell;
     b.nzero = (int64_t)ncopy * nword * g.ncell;
@@ -3400,7 +3410,7 @@ int lsc_from_profile(ocsc_ctx* c, double* r, int64_t ld, int64_t n, const long l
   k_lsc_profile<<<1, 1024, 0, st>>>(tot, c->lsc_plan, cur, bunch);
   k_lsc_spectrum<<<grid, 256, 0, st>>>(bunch, c->lsc_plan, Zr, Zi);
   k_lsc_wake<<<grid, 256, 0, st>>>(Zr, Zi, c->lsc_plan, W);
-  const int nblk = nred_blocks(c, n);
+  const int nblk = sm ? sm->nblk : nred_blocks(c, n);
   if (n > 0 && dr && sm)
     k_lsc_kick<true, true><<<nblk, kPT, 0, st>>>(r, ld, n, W, c->lsc_plan, dr->L, dr->r56, sm->sc, sm->part);
   else if (n > 0 && dr)

@@ -147,10 +147,12 @@ __device__ __forceinline__ void grid_coords(const double* xyz, const KickScalars
 //
 // What bounds them is latency: the trees sit at the end of every particle
 // pass and make up the single-workgroup kernels between the passes.  Inside a
-// wavefront values move by DPP (row shifts, then row broadcasts): a step is
-// two 4-cycle register moves per double where a shuffle is two trips through
-// the LDS pipe.  Measured (MI355X): the 11-value reduction kernel of a kick
-// 9.3 -> 3.3 us at 10 partials; see reduce_partials for the larger counts.
+// wavefront values move by lane swaps (32 and 16 lanes) and DPP row shifts (8,
+// 4, 2, 1): register moves, where a shuffle is a trip through the LDS pipe.
+// The tree is the shuffles' (lane i takes lane i + off, off halving), and the
+// wavefronts' results meet in a tree of the same shape: in the mixed form a
+// frame that differs in its last bit moves the FP32 rounding of every field
+// value, so the order of these sums is part of the result.
 template <int KIND>
 __device__ __forceinline__ double red_op(int c, double a, double b) {
   if (KIND == 1 && c < 3) return b < a ? b : a;
@@ -165,13 +167,20 @@ __device__ __forceinline__ double red_id(int c) {
   return 0.0;
 }
 
-// v of the lane that the DPP control CTRL reads from, `old` where it names
-// none (or the row is masked out)
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ double dpp_from(double v, double old) {
-  const int2 s = __builtin_bit_cast(int2, v), o = __builtin_bit_cast(int2, old);
-  const int2 r = {__builtin_amdgcn_update_dpp(o.x, s.x, CTRL, ROWS, 0xf, false),
-                  __builtin_amdgcn_update_dpp(o.y, s.y, CTRL, ROWS, 0xf, false)};
+// v of lane i + OFF, for lanes i < OFF (the lanes the tree reads)
+template <int OFF>
+__device__ __forceinline__ unsigned lane_above(unsigned v) {
+  if constexpr (OFF == 32)
+    return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  else if constexpr (OFF == 16)
+    return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  else
+    return __builtin_amdgcn_update_dpp(v, v, 0x100 + OFF, 0xf, 0xf, false);  // row_shl:OFF
+}
+template <int OFF>
+__device__ __forceinline__ double lane_above(double v) {
+  const uint2 s = __builtin_bit_cast(uint2, v);
+  const uint2 r = {lane_above<OFF>(s.x), lane_above<OFF>(s.y)};
   return __builtin_bit_cast(double, r);
 }
 
@@ -182,24 +191,22 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
 }
 
 // NV values reduced over the 64 lanes of a wavefront (all of them active);
-// the results are uniform.  c0: the component of v[0] (KIND 1)
+// the results are in lane 0
 template <int NV, int KIND>
-__device__ __forceinline__ void wave_reduce(double* v, int c0 = 0) {
-#define OCSC_RED_STEP(CTRL, ROWS)                                                                          \
-  _Pragma("unroll") for (int c = 0; c < NV; ++c) v[c] =                                                    \
-      red_op<KIND>(c0 + c, v[c], dpp_from<CTRL, ROWS>(v[c], red_id<KIND>(c0 + c)))
-  OCSC_RED_STEP(0x111, 0xf);  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row
-  OCSC_RED_STEP(0x112, 0xf);
-  OCSC_RED_STEP(0x114, 0xf);
-  OCSC_RED_STEP(0x118, 0xf);
-  OCSC_RED_STEP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
-  OCSC_RED_STEP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3: lane 63 holds the wavefront
+__device__ __forceinline__ void wave_reduce(double* v) {
+#define OCSC_RED_STEP(OFF) \
+  _Pragma("unroll") for (int c = 0; c < NV; ++c) v[c] = red_op<KIND>(c, v[c], lane_above<OFF>(v[c]))
+  OCSC_RED_STEP(32);
+  OCSC_RED_STEP(16);
+  OCSC_RED_STEP(8);
+  OCSC_RED_STEP(4);
+  OCSC_RED_STEP(2);
+  OCSC_RED_STEP(1);
 #undef OCSC_RED_STEP
-#pragma unroll
-  for (int c = 0; c < NV; ++c) v[c] = lane_value(v[c], 63);
 }
 
-// result valid in the first wavefront; lds holds (blockDim/64) * NV doubles
+// result valid in the first wavefront; lds holds (blockDim/64) * NV doubles,
+// at most 16 wavefronts
 template <int NV, int KIND>
 __device__ __forceinline__ void block_reduce(double* v, double* lds) {
   static_assert(NV <= 64, "one lane per value");
@@ -209,44 +216,96 @@ __device__ __forceinline__ void block_reduce(double* v, double* lds) {
 #pragma unroll
     for (int c = 0; c < NV; ++c) lds[w * NV + c] = v[c];
   __syncthreads();
-  // lane c adds the wavefronts' values of component c in order
+  // lane c takes component c through the tree over the wavefronts
   if (w == 0) {
     const int c0 = lane < NV ? lane : 0;
-    double t = lds[c0];
-    for (int k = 1; k < nw; ++k) t = red_op<KIND>(c0, t, lds[k * NV + c0]);
+    double t;
+    if (nw == 4) {
+      const double u0 = red_op<KIND>(c0, lds[c0], lds[2 * NV + c0]);
+      const double u1 = red_op<KIND>(c0, lds[NV + c0], lds[3 * NV + c0]);
+      t = red_op<KIND>(c0, u0, u1);
+    } else {
+      double u[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) u[k] = k < nw ? lds[k * NV + c0] : red_id<KIND>(c0);
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < off; ++k) u[k] = red_op<KIND>(c0, u[k], u[k + off]);
+      t = u[0];
+    }
 #pragma unroll
     for (int c = 0; c < NV; ++c) v[c] = lane_value(t, c);
   }
 }
 
+// One component's nblk partials through the tree of a 1024-thread workgroup
+// (thread t adds partials t, t + 1024, ... in order; then lanes; then
+// wavefronts) by one wavefront: value w of lane l stands for thread l + 64 w.
+// Four values at a time go through the lanes as independent chains; their
+// results wait in lds[0..16) and lane w then takes value w.  The loop stays
+// rolled: these kernels run once per kick, from a cold instruction cache, and
+// 16 unrolled chains per component were no faster than the shuffles.  OP 0
+// sum, 1 minimum, 2 maximum; result in lane 0.
+template <int OP>
+__device__ __forceinline__ double partials_total(const double* __restrict__ p, int nblk, double* lds) {
+  constexpr int KIND = OP ? 1 : 0, C = OP == 2 ? 3 : 0, G = 4;
+  const int lane = threadIdx.x & 63;
+  const int nw = nblk < 1024 ? (nblk + 63) >> 6 : 16;
+#pragma unroll 1
+  for (int w0 = 0; w0 < nw; w0 += G) {
+    double t[G];
+    const int b = lane + 64 * w0;
+#pragma unroll
+    for (int k = 0; k < G; ++k) t[k] = b + 64 * k < nblk ? p[b + 64 * k] : red_id<KIND>(C);
+#pragma unroll 1
+    for (int b1 = b + 1024; b1 < nblk; b1 += 1024)
+#pragma unroll
+      for (int k = 0; k < G; ++k)
+        if (b1 + 64 * k < nblk) t[k] = red_op<KIND>(C, t[k], p[b1 + 64 * k]);
+#define OCSC_RED_STEP(OFF) \
+  _Pragma("unroll") for (int k = 0; k < G; ++k) t[k] = red_op<KIND>(C, t[k], lane_above<OFF>(t[k]))
+    OCSC_RED_STEP(32);
+    OCSC_RED_STEP(16);
+    OCSC_RED_STEP(8);
+    OCSC_RED_STEP(4);
+    OCSC_RED_STEP(2);
+    OCSC_RED_STEP(1);
+#undef OCSC_RED_STEP
+    if (lane == 0)
+#pragma unroll
+      for (int k = 0; k < G; ++k) lds[w0 + k] = t[k];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // lane 0's stores before the lanes' loads
+  __builtin_amdgcn_wave_barrier();
+  double v = lane < nw ? lds[lane & 15] : red_id<KIND>(C);
+  v = red_op<KIND>(C, v, lane_above<8>(v));
+  v = red_op<KIND>(C, v, lane_above<4>(v));
+  v = red_op<KIND>(C, v, lane_above<2>(v));
+  return red_op<KIND>(C, v, lane_above<1>(v));
+}
+
 // Totals of nblk partials of NV components, stored transposed (part[c * nblk
-// + b], coalesced): a wavefront takes whole components, its lanes adding
-// every 64th partial (U loads in flight, added in increasing b), so a
-// component needs one wavefront reduction instead of one per wavefront of the
-// workgroup.  out is valid in every thread; lds holds NV doubles.  The 11
-// components of 977 partials: 10.7 -> 5.2 us, 12 of 2048: 10.0 -> 5.0 us (a
-// workgroup of 16 wavefronts, each reducing every component by shuffles,
-// before).
+// + b], coalesced), in every thread; lds holds 16 * NV doubles.  A wavefront
+// takes whole components, so a component needs no workgroup barrier of its
+// own and the code is one short loop.
 template <int NV, int KIND>
 __device__ __forceinline__ void reduce_partials(const double* __restrict__ part, int nblk, double* out, double* lds) {
-  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  constexpr int U = 8;
-  for (int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); c < NV; c += nw) {
-    double v = red_id<KIND>(c);
+#pragma unroll 1
+  for (int c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); c < NV; c += blockDim.x >> 6) {
     const double* p = part + (int64_t)c * nblk;
-    for (int b0 = lane; b0 < nblk; b0 += U * 64) {
-      double t[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) t[u] = b0 + u * 64 < nblk ? p[b0 + u * 64] : red_id<KIND>(c);
-#pragma unroll
-      for (int u = 0; u < U; ++u) v = red_op<KIND>(c, v, t[u]);
-    }
-    wave_reduce<1, KIND>(&v, c);
-    if (lane == 0) lds[c] = v;
+    double v;
+    if (KIND == 1 && c < 3)
+      v = partials_total<1>(p, nblk, lds + 16 * c);
+    else if (KIND == 1 && c < 6)
+      v = partials_total<2>(p, nblk, lds + 16 * c);
+    else
+      v = partials_total<0>(p, nblk, lds + 16 * c);
+    if ((threadIdx.x & 63) == 0) lds[16 * c] = v;
   }
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < NV; ++c) out[c] = lds[c];
+  for (int c = 0; c < NV; ++c) out[c] = lds[16 * c];
 }
 
 // First level of a two-level sum over many block partials: block f of the
@@ -322,7 +381,7 @@ __global__ void __launch_bounds__(kPT) k_passA(Rows R, KickScalars* __restrict__
 // frame from the mean momentum (sc.py:224-239)
 __device__ __forceinline__ void reduceA_body(KickScalars* __restrict__ scp, const double* __restrict__ part, int nblk,
                                              const int bx, const int nbx) {
-  __shared__ double lds[3];
+  __shared__ double lds[16 * 3];
   double acc[3];
   reduce_partials<3, 0>(part, nblk, acc, lds);
   if (threadIdx.x != 0) return;
@@ -435,7 +494,7 @@ __global__ void __launch_bounds__(kPT) k_passB(Rows R, const double* __restrict_
 // (sc.py:172-186)
 __device__ __forceinline__ void reduceB_body(KickScalars* __restrict__ scp, const double* __restrict__ part, int nblk,
                                              int prec, const int bx, const int nbx) {
-  __shared__ double tot[kNPartB];
+  __shared__ double tot[16 * kNPartB];
   double out[kNPartB];
   reduce_partials<kNPartB, 1>(part, nblk, out, tot);
   if (threadIdx.x >= 64) return;
@@ -447,7 +506,7 @@ __device__ __forceinline__ void reduceB_body(KickScalars* __restrict__ scp, cons
   bool same = true;
   double h = 0;
   if (k < 3) {
-    const double xmin = tot[k], xmax = tot[3 + k], sumqx = tot[8 + k];
+    const double xmin = tot[16 * k], xmax = tot[16 * (3 + k)], sumqx = tot[16 * (8 + k)];
     s.xmin[k] = xmin;
     s.xmax[k] = xmax;
     s.sumqx[k] = sumqx;
