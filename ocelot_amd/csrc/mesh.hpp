@@ -75,9 +75,9 @@ __device__ __forceinline__ double charge_at(const void* src, int64_t i, int64_t 
   } else {
     const long long* a = (const long long*)src;
     unsigned long long hi = 0, lo = 0;
-    for (int c = 0; c < ncopy; ++c) {
-      hi += (unsigned long long)a[2 * c * ncell + i];
-      lo += (unsigned long long)a[(2 * c + 1) * ncell + i];
+    for (int c = 0; c < ncopy; ++c) {  // a cell's two words lie side by side
+      hi += (unsigned long long)a[2 * (c * ncell + i)];
+      lo += (unsigned long long)a[2 * (c * ncell + i) + 1];
     }
     return ((double)(long long)hi + (double)(long long)lo * 0x1p-30) * inv_qscale;
   }

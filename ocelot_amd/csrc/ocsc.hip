@@ -752,6 +752,7 @@ struct StepOpts {
   // z pass, its last reader, runs before the kick)
   bool grid_zeroed = false;
   bool zero_next = false;
+  bool ordered = false;  // the rows are in cell order (the copy of a tracking call)
 };
 
 // buffers of a kick on a cell-ordered copy: sort keys and values (ping-pong),
@@ -779,12 +780,29 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
   k_deposit<NWORD, XCD, AGG, TILE><<<(int)((n + per - 1) / per), kDepPT, 0, st>>>(R, q, sc, grid, cells);
 }
 
+// The tile the default (option deposit_tile 0, no other deposit option) takes.
+// In the caller's order a workgroup's particles share few cells, so the table
+// only delays its atomics: without it 20k / 31^3 FP64 148 -> 120 us per kick
+// (10 workgroups of 8 particles per thread left the chip idle), 200k / 63^3
+// 177 -> 158, 1.5M / 63^3 403 -> 358, 4M / 127^3 mixed 873 -> 856.  One particle
+// per thread up to 150k (100k: 147 either way, 200k: 162 with one, 158 with
+// eight).  In cell order the table pays (2M / 63^3 FP64 tracking step 224 us
+// with it, 351 without), at two particles per thread (231 with eight).
+constexpr int64_t kDepOneMax = 150000;
+int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered) {
+  if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
+  if (ordered) return 6;
+  return n <= kDepOneMax ? 5 : 3;
+}
+
 // the deposit variant the context's options select
 template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
-                    int32_t* cells, int64_t n, hipStream_t st) {
+                    int32_t* cells, int64_t n, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = c->deposit_tile;
+  const int t = dep_tile(c, n, ordered);
+  if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
+  if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \
   if (v == V && t == T) return launch_deposit_t<NWORD, (V & 4) != 0, (V & 2) != 0, T>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP3(V) OCSC_DEP(V, 0) OCSC_DEP(V, 1) OCSC_DEP(V, 2) OCSC_DEP(V, 3) OCSC_DEP(V, 4)
@@ -917,11 +935,11 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
     }
   }
   if (rec_direct) {
-    constexpr int per = kDepPT * DepTile<0>::items;
-    k_deposit<NWORD, false, false, 0, true><<<(int)((n + per - 1) / per), kDepPT, 0, st>>>(
+    constexpr int per = kDepPT * DepTile<6>::items;
+    k_deposit<NWORD, false, false, 6, true><<<(int)((n + per - 1) / per), kDepPT, 0, st>>>(
         R, q, L.sc, (unsigned long long*)L.grid.p, nullptr, sb->rec, order);
   } else {
-    launch_deposit<NWORD>(c, R, q, L.sc, (unsigned long long*)L.grid.p, o.cells, n, st);
+    launch_deposit<NWORD>(c, R, q, L.sc, (unsigned long long*)L.grid.p, o.cells, n, o.ordered || sb, st);
   }
   LAUNCHCHK("deposit");
   mark(3);
@@ -2071,6 +2089,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
       o.prev_nblk = frame_blocks(c, n, prec);
     }
     o.dr = DriftArgs{Ld, r56};
+    o.ordered = sorted;
     o.grid_zeroed = c->grid_clear == 2 && step > 0;
     o.zero_next = c->grid_clear == 2 && step < nsteps - 1;
     if (ktime) {

@@ -625,23 +625,42 @@ constexpr int kDepSlots2 = 1024;             // two-word (FP64) form: half the L
 // probes a nearly full table before it falls through), 4 as 0 with the rows
 // of all of a thread's particles loaded before the first is deposited (tile
 // 0 loads one particle ahead; the deposit waits on memory most of its time)
+// Not options: tiles that the default (0) takes by itself, 5 one particle per
+// thread and no table, 6 a quarter of tile 0 (see dep_tile).
 template <int TILE>
 struct DepTile {
-  static constexpr bool direct = TILE == 3;
+  static constexpr bool direct = TILE == 3 || TILE == 5;
   static constexpr bool all_loads = TILE == 4;  // as 0, every item's loads issued first
-  static constexpr int items = TILE == 1 ? kDepItems / 2 : (TILE == 2 ? kDepItems * 2 : kDepItems);
+  static constexpr int items =
+      TILE == 1 ? kDepItems / 2 : (TILE == 2 ? kDepItems * 2 : (TILE == 5 ? 1 : (TILE == 6 ? kDepItems / 4 : kDepItems)));
   template <int NWORD>
   static constexpr int slots() {
     constexpr int base = NWORD == 2 ? kDepSlots2 : kDepSlots;
-    return TILE == 1 ? base / 2 : (TILE == 2 ? base * 2 : (TILE == 3 ? 1 : base));
+    return TILE == 1 ? base / 2 : (TILE == 2 ? base * 2 : (direct ? 1 : (TILE == 6 ? base / 4 : base)));
   }
 };
 
+// a cell's words lie side by side: [cell][NWORD]
 template <bool XCD>
-__device__ __forceinline__ void flush_cell(unsigned long long* g, int64_t ncell, int64_t idx, long long hi,
-                                           long long lo, int nword) {
-  grid_add<XCD>(g, idx, hi);
-  if (nword == 2) grid_add<XCD>(g, ncell + idx, lo);
+__device__ __forceinline__ void flush_cell(unsigned long long* g, int64_t idx, long long hi, long long lo, int nword) {
+  grid_add<XCD>(g, nword * idx, hi);
+  if (nword == 2) grid_add<XCD>(g, nword * idx + 1, lo);
+}
+
+// Two words per cell, every lane of the wavefront with a cell (or -1) of its
+// own: lane pairs take the two words of one particle, then of the other, so an
+// atomic instruction carries 32 pairs of neighbouring words (one request each)
+// where a lane adding both of its words sends 64 requests twice.
+template <bool XCD>
+__device__ __forceinline__ void flush_pairs(unsigned long long* g, int idx, long long hi, long long lo) {
+  const int lane = threadIdx.x & 63, odd = lane & 1;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int src = (lane & ~1) | h;
+    const int i = __shfl(idx, src);
+    const long long vh = __shfl(hi, src), vl = __shfl(lo, src);
+    if (i >= 0) grid_add<XCD>(g, 2 * (int64_t)i + odd, odd ? vl : vh);
+  }
 }
 
 // cells (may be null): receives the flat cell index each particle's charge
@@ -650,8 +669,8 @@ __device__ __forceinline__ void flush_cell(unsigned long long* g, int64_t ncell,
 // probing; cell indices fit in 31 bits: mesh <= 1024^3), or straight to the
 // grid when the table is crowded
 template <int NWORD, bool XCD, int kSlots>
-__device__ __forceinline__ void hash_add(int* hkey, long long (*hval)[kSlots], unsigned long long* g, int64_t ncell,
-                                         int64_t idx, long long hi, long long lo) {
+__device__ __forceinline__ void hash_add(int* hkey, long long (*hval)[kSlots], unsigned long long* g, int64_t idx,
+                                         long long hi, long long lo) {
   unsigned slot = ((unsigned)idx * 2654435761u) >> (32 - ilog2(kSlots));
   for (int probe = 0; probe < 32; ++probe) {
     const int k = atomicCAS(&hkey[slot], -1, (int)idx);
@@ -662,7 +681,7 @@ __device__ __forceinline__ void hash_add(int* hkey, long long (*hval)[kSlots], u
     }
     slot = (slot + 1) & (kSlots - 1);
   }
-  flush_cell<XCD>(g, ncell, idx, hi, lo, NWORD);
+  flush_cell<XCD>(g, idx, hi, lo, NWORD);
 }
 
 // Wave-level pre-sum (AGG): in cell order, neighbouring lanes usually carry
@@ -688,6 +707,7 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
   unsigned long long* g = grid;
   if constexpr (XCD) g += (int64_t)xcc_id() * NWORD * ncell;
   constexpr bool kDirect = DepTile<TILE>::direct;
+  constexpr bool kPairs = kDirect && NWORD == 2 && !AGG;
   if constexpr (!kDirect) {
     for (int i = threadIdx.x; i < kSlots; i += kDepPT) {
       hkey[i] = -1;
@@ -747,15 +767,17 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
       const int knext = __shfl_down(key, 1);
       if (key >= 0 && (lane == 63 || knext != key)) {
         if constexpr (kDirect)
-          flush_cell<XCD>(g, ncell, key, hi, lo, NWORD);
+          flush_cell<XCD>(g, key, hi, lo, NWORD);
         else
-          hash_add<NWORD, XCD, kSlots>(hkey, hval, g, ncell, key, hi, lo);
+          hash_add<NWORD, XCD, kSlots>(hkey, hval, g, key, hi, lo);
       }
+    } else if constexpr (kPairs) {
+      flush_pairs<XCD>(g, (int)idx, hi, lo);
     } else if (idx >= 0) {
       if constexpr (kDirect)
-        flush_cell<XCD>(g, ncell, idx, hi, lo, NWORD);
+        flush_cell<XCD>(g, idx, hi, lo, NWORD);
       else
-        hash_add<NWORD, XCD, kSlots>(hkey, hval, g, ncell, idx, hi, lo);
+        hash_add<NWORD, XCD, kSlots>(hkey, hval, g, idx, hi, lo);
     }
   };
   if constexpr (DepTile<TILE>::all_loads) {
@@ -770,8 +792,8 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
     for (int it = 0; it < kItems; ++it) {
       const int64_t p = base + threadIdx.x + (int64_t)it * kDepPT;
       const bool valid = p < s.n;
-      if constexpr (AGG) {
-        if (__ballot(valid) == 0) break;  // uniform across the wave: every lane takes part in the scan
+      if constexpr (AGG || kPairs) {
+        if (__ballot(valid) == 0) break;  // uniform across the wave: every lane takes part
       } else {
         if (!valid) break;
       }
@@ -784,8 +806,8 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
     if (p < s.n) load(p, cur);
     for (int it = 0; it < kItems; ++it, p += kDepPT) {
       const bool valid = p < s.n;
-      if constexpr (AGG) {
-        if (__ballot(valid) == 0) break;  // uniform across the wave: every lane takes part in the scan
+      if constexpr (AGG || kPairs) {
+        if (__ballot(valid) == 0) break;  // uniform across the wave: every lane takes part
       } else {
         if (!valid) break;
       }
@@ -801,9 +823,10 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
   if (bad) atomicOr(&scp->err, (int)kErrCell);
   if constexpr (!kDirect) {
     __syncthreads();
-    for (int i = threadIdx.x; i < kSlots; i += kDepPT) {
-      const int k = hkey[i];
-      if (k >= 0) flush_cell<XCD>(g, ncell, k, hval[0][i], NWORD == 2 ? hval[NWORD - 1][i] : 0, NWORD);
+    // neighbouring threads take the words of one slot (one request per cell)
+    for (int i = threadIdx.x; i < NWORD * kSlots; i += kDepPT) {
+      const int k = hkey[i / NWORD];
+      if (k >= 0) grid_add<XCD>(g, NWORD * (int64_t)k + i % NWORD, hval[i % NWORD][i / NWORD]);
     }
   }
 }
@@ -1435,7 +1458,6 @@ __global__ void __launch_bounds__(kPT) k_deposit_xyz(Rows R, const double* __res
   if (s0.err) return;
   const KickScalars s = s0;
   const int nx = s.nmesh[0], ny = s.nmesh[1], nz = s.nmesh[2];
-  const int64_t ncell = (int64_t)nx * ny * nz;
   const int64_t p = (int64_t)blockIdx.x * kPT + threadIdx.x;
   if (p >= s.n) return;
   double xyz[3] = {R.r[p], R.r[R.ld + p], R.r[2 * R.ld + p] * s.gamma0}, X[3];
@@ -1448,10 +1470,10 @@ __global__ void __launch_bounds__(kPT) k_deposit_xyz(Rows R, const double* __res
   const int64_t idx = ((int64_t)f0 * ny + (int64_t)f1) * nz + (int64_t)f2;
   const double v = q[p] * s.qscale;
   const double hi = __builtin_rint(v);
-  atomicAdd(&grid[idx], (unsigned long long)(long long)hi);
+  atomicAdd(&grid[NWORD * idx], (unsigned long long)(long long)hi);
   if constexpr (NWORD == 2) {
     const double lo = __builtin_rint((v - hi) * 0x1p30);
-    atomicAdd(&grid[ncell + idx], (unsigned long long)(long long)lo);
+    atomicAdd(&grid[NWORD * idx + 1], (unsigned long long)(long long)lo);
   }
 }
 
