@@ -193,7 +193,7 @@ __global__ void __launch_bounds__((pass_threads<float, M, V>())) kb_zinv3(const 
   OCSC_BJOB();
   (void)nbx;
   const int64_t nyz = (int64_t)b.d.nx * b.d.ny * b.d.hz;
-  zinv3_body<M, V>((const cpx<float>*)b.A, nyz, (float*)b.phi, b.ncell, b.d, b.sc, tw, twd, blockIdx.y, bx);
+  zinv3_body<M, V>((const cpx<float>*)b.A, nyz, (float*)b.phi, b.ncell, false, b.d, b.sc, tw, twd, blockIdx.y, bx);
 }
 
 // FP64 form: convolution to the potential, then the difference fields

@@ -555,12 +555,49 @@ __global__ void __launch_bounds__((pass_threads<F, M, V>())) k_yinv(const cpx<F>
   yinv_body<F, M, V>(B, A, d, sc, tw, blockIdx.x, gridDim.x);
 }
 
+// Line layout of the fields, for kicks in the caller's (random) order.  A
+// particle reads the three components around one place of the mesh, 2 x 2 rows
+// along z each and two neighbours of every row.  From one grid per component
+// that is 12 lines of 128 bytes; here a line holds the three components of KB
+// consecutive planes of one row, and the next two planes over again (a
+// component sampled half a cell on starts up to one plane further, and reads a
+// pair), so a particle touches 4 to 8 lines:
+//   line (row, z / KB), component c, plane z: word c (KB + 2) + z % KB
+// FP32: KB = 8, 30 of 32 words; FP64: KB = 3, 15 of 16 words.  50M particles
+// on 255^3 mixed: kick 16.0 -> 10.7 ms; 10M on 127^3 FP64, hollow bunch: 3.29
+// -> 2.28 ms.  In cell order neighbouring particles share the grids' lines and
+// the larger array costs (2M / 63^3 FP64 tracking step 221 us from the grids,
+// 229 from lines), so cell-ordered kicks keep one grid per component.
+template <typename F>
+struct FieldLine {
+  static constexpr int KB = sizeof(F) == 4 ? 8 : 3;
+  static constexpr int CW = KB + 2;             // words per component
+  static constexpr int W = 128 / (int)sizeof(F);  // words per line
+  static_assert(3 * CW <= W, "three components in a line");
+  __host__ __device__ static constexpr int per_row(int nz) { return (nz + KB - 1) / KB; }
+  __host__ __device__ static constexpr size_t bytes(int nx, int ny, int nz) {
+    return (size_t)nx * ny * per_row(nz) * 128;
+  }
+};
+
+// value v of component comp at (row, z), at both of its places
+template <typename F>
+__device__ __forceinline__ void store_field(F* __restrict__ E, int64_t row, int z, int nz, int comp, F v) {
+  using L = FieldLine<F>;
+  const int b = z / L::KB, k = z - b * L::KB;
+  F* const at = E + (row * L::per_row(nz) + b) * L::W + comp * L::CW + k;
+  *at = v;
+  if (k < 2 && b > 0) at[L::KB - L::W] = v;
+}
+
 // z pass inverse: two Hermitian half spectra -> one complex inverse FFT ->
-// two real rows of the potential, z < nz
+// two real rows of the potential, z < nz (comp >= 0: of that component's field,
+// in the line layout)
 template <typename F, int M, bool DERIV, int V = 0>
 __device__ __forceinline__ void zinv_rows(const cpx<F>* __restrict__ A, F* __restrict__ phi, const MeshDims& d,
                                           const KickScalars* __restrict__ sc, const cpx<F>* __restrict__ tw,
-                                          const cpx<double>* __restrict__ twd, cpx<F>* s, const int bx) {
+                                          const cpx<double>* __restrict__ twd, cpx<F>* s, const int bx,
+                                          const int comp = -1) {
   using TL = Tile<F, M, V>;
   constexpr int T = TL::T, S = TL::S;
   const cpx<F>* twl = stage_tw<F, M, kNT, TL::stw>(s + (size_t)M * S, tw);
@@ -607,7 +644,11 @@ __device__ __forceinline__ void zinv_rows(const cpx<F>* __restrict__ A, F* __res
     const int64_t row = row0 + rl;
     if (row >= R) continue;
     const cpx<F> v = s[z * S + (rl >> 1)];
-    phi[row * nz + z] = (rl & 1) ? v.y : v.x;
+    const F w = (rl & 1) ? v.y : v.x;
+    if (comp < 0)
+      phi[row * nz + z] = w;
+    else
+      store_field(phi, row, z, nz, comp, w);
   }
 }
 
@@ -619,7 +660,8 @@ __device__ __forceinline__ void zinv_rows(const cpx<F>* __restrict__ A, F* __res
 template <typename F, int M, bool DERIV>
 __device__ __forceinline__ void zinv_rows_reg(const cpx<F>* __restrict__ A, F* __restrict__ phi, const MeshDims& d,
                                               const KickScalars* __restrict__ sc, const cpx<F>* __restrict__ tw,
-                                              const cpx<double>* __restrict__ twd, cpx<F>* s, const int bx) {
+                                              const cpx<double>* __restrict__ twd, cpx<F>* s, const int bx,
+                                              const int comp = -1) {
   constexpr int R = reg_r<M>(), Q = reg_q<M>(), T = Tile<F, M>::T, NT = Q * T;
   cpx<F>* twl = s + RegX<R, Q, T>::entries;
   cpx<F>* dl = twl + M;
@@ -661,8 +703,13 @@ __device__ __forceinline__ void zinv_rows_reg(const cpx<F>* __restrict__ A, F* _
   for (int q = 0; q < R / 2; ++q) {
     const int z = j + Q * q;
     if (z < nz) {
-      if (ra < nrow) phi[ra * nz + z] = x[q].x;
-      if (rb < nrow) phi[rb * nz + z] = x[q].y;
+      if (comp < 0) {
+        if (ra < nrow) phi[ra * nz + z] = x[q].x;
+        if (rb < nrow) phi[rb * nz + z] = x[q].y;
+      } else {
+        if (ra < nrow) store_field(phi, ra, z, nz, comp, x[q].x);
+        if (rb < nrow) store_field(phi, rb, z, nz, comp, x[q].y);
+      }
     }
   }
 }
@@ -689,34 +736,36 @@ __global__ void __launch_bounds__((pass_threads<F, M, V>())) k_zinv(const cpx<F>
 }
 
 // Mixed form: the three field components in one launch (blockIdx.y), the
-// third (z) with the spectral difference factor
+// third (z) with the spectral difference factor; one grid after the other at E,
+// or in the line layout (lines)
 template <int M, int V>
 __device__ __forceinline__ void zinv3_body(const cpx<float>* __restrict__ A, int64_t nyz, float* __restrict__ E,
-                                           int64_t ncell, const MeshDims& d, const KickScalars* __restrict__ sc,
+                                           int64_t ncell, bool lines, const MeshDims& d, const KickScalars* __restrict__ sc,
                                            const cpx<float>* __restrict__ tw, const cpx<double>* __restrict__ twd,
                                            const int comp, const int bx) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   if (sc->err) return;
   cpx<float>* s = (cpx<float>*)smem_raw;
+  float* const E2 = lines ? E : E + comp * ncell;
   if constexpr (reg_plan<float, M, V>()) {
     if (comp == 2)
-      zinv_rows_reg<float, M, true>(A + 2 * nyz, E + 2 * ncell, d, sc, tw, twd, s, bx);
+      zinv_rows_reg<float, M, true>(A + 2 * nyz, E2, d, sc, tw, twd, s, bx, lines ? 2 : -1);
     else
-      zinv_rows_reg<float, M, false>(A + comp * nyz, E + comp * ncell, d, sc, tw, twd, s, bx);
+      zinv_rows_reg<float, M, false>(A + comp * nyz, E2, d, sc, tw, twd, s, bx, lines ? comp : -1);
   } else {
     if (comp == 2)
-      zinv_rows<float, M, true, V>(A + 2 * nyz, E + 2 * ncell, d, sc, tw, twd, s, bx);
+      zinv_rows<float, M, true, V>(A + 2 * nyz, E2, d, sc, tw, twd, s, bx, lines ? 2 : -1);
     else
-      zinv_rows<float, M, false, V>(A + comp * nyz, E + comp * ncell, d, sc, tw, twd, s, bx);
+      zinv_rows<float, M, false, V>(A + comp * nyz, E2, d, sc, tw, twd, s, bx, lines ? comp : -1);
   }
 }
 
 template <int M, int V = 0>
 __global__ void __launch_bounds__((pass_threads<float, M, V>())) k_zinv3(const cpx<float>* __restrict__ A, int64_t nyz, float* __restrict__ E,
-                                               int64_t ncell, MeshDims d, const KickScalars* __restrict__ sc,
+                                               int64_t ncell, int lines, MeshDims d, const KickScalars* __restrict__ sc,
                                                const cpx<float>* __restrict__ tw,
                                                const cpx<double>* __restrict__ twd) {
-  zinv3_body<M, V>(A, nyz, E, ncell, d, sc, tw, twd, blockIdx.y, blockIdx.x);
+  zinv3_body<M, V>(A, nyz, E, ncell, lines != 0, d, sc, tw, twd, blockIdx.y, blockIdx.x);
 }
 
 // columns per workgroup of the kernels that carry two or three fields

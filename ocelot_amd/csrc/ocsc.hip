@@ -591,11 +591,11 @@ int launch_convolution(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho,
 
 // Mixed form: the three field components on the mesh, E = -grad phi as the
 // forward differences of the reference (sc.py:195-200) taken in Fourier
-// space, written as three FP32 grids one after the other at E.  V: the FFT
-// plan variant (option "fft_plan").
+// space, written as three FP32 grids one after the other at E, or in the line
+// layout (lines).  V: the FFT plan variant (option "fft_plan").
 template <int V>
-int launch_fields_v(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho, float* E, hipStream_t st,
-                    hipEvent_t* ev, hipEvent_t join) {
+int launch_fields_v(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho, float* E, bool lines,
+                    hipStream_t st, hipEvent_t* ev, hipEvent_t join) {
   const MeshDims& d = g.d;
   const int64_t nyz = (int64_t)d.nx * d.ny * d.hz;
   cpx<float>* A = (cpx<float>*)L.A.p;
@@ -639,25 +639,25 @@ int launch_fields_v(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho, fl
     using TL = Tile<float, MM, V>;
     const int nb = (int)((R + 2 * TL::T - 1) / (2 * TL::T));
     k_zinv3<MM, V><<<dim3(nb, 3), pass_threads<float, MM, V>(), pass_lds<float, MM, V>(), st>>>(
-        A, nyz, E, g.ncell, d, L.sc, c->twf + MM, c->twd + MM);
+        A, nyz, E, g.ncell, lines ? 1 : 0, d, L.sc, c->twf + MM, c->twd + MM);
   });
   LAUNCHCHK("k_zinv(fields)");
   return OCSC_OK;
 }
 
-int launch_fields(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho, float* E, hipStream_t st,
-                  hipEvent_t* ev = nullptr, hipEvent_t join = nullptr) {
+int launch_fields(ocsc_ctx* c, Lane& L, const Geometry& g, const void* rho, float* E, bool lines,
+                  hipStream_t st, hipEvent_t* ev = nullptr, hipEvent_t join = nullptr) {
   switch (c->fft_plan) {
     case 1:
-      return launch_fields_v<1>(c, L, g, rho, E, st, ev, join);
+      return launch_fields_v<1>(c, L, g, rho, E, lines, st, ev, join);
     case 2:
-      return launch_fields_v<2>(c, L, g, rho, E, st, ev, join);
+      return launch_fields_v<2>(c, L, g, rho, E, lines, st, ev, join);
     case 3:
-      return launch_fields_v<3>(c, L, g, rho, E, st, ev, join);
+      return launch_fields_v<3>(c, L, g, rho, E, lines, st, ev, join);
     case 4:
-      return launch_fields_v<4>(c, L, g, rho, E, st, ev, join);
+      return launch_fields_v<4>(c, L, g, rho, E, lines, st, ev, join);
     default:
-      return launch_fields_v<0>(c, L, g, rho, E, st, ev, join);
+      return launch_fields_v<0>(c, L, g, rho, E, lines, st, ev, join);
   }
 }
 
@@ -753,6 +753,7 @@ struct StepOpts {
   bool grid_zeroed = false;
   bool zero_next = false;
   bool ordered = false;  // the rows are in cell order (the copy of a tracking call)
+  bool lines = false;    // the fields in the line layout (FieldLine; buffers sized for it by the caller)
 };
 
 // buffers of a kick on a cell-ordered copy: sort keys and values (ping-pong),
@@ -778,6 +779,22 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
                       hipStream_t st) {
   constexpr int per = kDepPT * DepTile<TILE>::items;
   k_deposit<NWORD, XCD, AGG, TILE><<<(int)((n + per - 1) / per), kDepPT, 0, st>>>(R, q, sc, grid, cells);
+}
+
+// The line layout of the fields pays from about one particle per two cells
+// (mixed: 250k / 63^3 177 -> 167 us, 2M / 127^3 hollow 760 -> 551), in the FP64
+// form, with 1.8 times the grids' bytes, where the grids are larger than the
+// L2s hold (2M / 63^3, 6 MB: 354 us either way; 5M / 127^3, 49 MB: 1001 ->
+// 965, hollow 1697 -> 1269).  Where the larger array is refused: the grids.
+bool line_fields(Lane& L, const Geometry& g, int64_t n, int prec) {
+  const MeshDims& d = g.d;
+  if (2 * n < g.ncell || (prec == OCSC_FP64 && g.ncell * 24 < (16 << 20))) return false;
+  Buf& b = prec == OCSC_FP64 ? L.E64 : L.phi;
+  const size_t grids = b.cap, lines = prec == OCSC_FP64 ? FieldLine<double>::bytes(d.nx, d.ny, d.nz)
+                                                        : FieldLine<float>::bytes(d.nx, d.ny, d.nz);
+  if (ensure(b, lines) == OCSC_OK) return true;
+  (void)ensure(b, grids);  // what it had
+  return false;
 }
 
 // The tile the default (option deposit_tile 0, no other deposit option) takes.
@@ -814,7 +831,7 @@ void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc,
 template <typename F, bool DRIFT, bool SUMP>
 void launch_kick(ocsc_ctx* c, Lane& L, int npart, double* r, int64_t ld, const StepOpts& o, int64_t nz64,
                  hipStream_t st) {
-  // mixed form: the three FP32 field grids; FP64 form: the k_diff64 fields
+  // mixed form: the three FP32 fields; FP64 form: the k_diff64 fields
   const F* field = sizeof(F) == 8 ? (const F*)L.E64.p : (const F*)L.phi.p;
   unsigned long long* zg = o.zero_next ? (unsigned long long*)L.grid.p : nullptr;
   if (!DRIFT && !SUMP && o.rec_out && o.rec_in)
@@ -823,6 +840,8 @@ void launch_kick(ocsc_ctx* c, Lane& L, int npart, double* r, int64_t ld, const S
   else if (!DRIFT && !SUMP && o.rec_out)
     k_kick<F, false, false, true><<<npart, kKickPT, 0, st>>>(r, ld, field, L.sc, o.dr, (double*)L.part.p, o.rec_perm,
                                                              o.rec_out, zg, zg ? nz64 : 0);
+  else if (!DRIFT && !SUMP && o.lines)
+    k_kick<F, false, false, false, false, true><<<npart, kKickPT, 0, st>>>(r, ld, field, L.sc, o.dr);
   else
     k_kick<F, DRIFT, SUMP><<<npart, kKickPT, 0, st>>>(r, ld, field, L.sc, o.dr, (double*)L.part.p, nullptr, nullptr,
                                                       zg, zg ? nz64 : 0);
@@ -946,7 +965,7 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   if (!fork && (rc = launch_kernel_spectrum<F>(c, L, g, st, 0))) return rc;
   mark(4);
   if constexpr (sizeof(F) == 4) {
-    if ((rc = launch_fields(c, L, g, L.grid.p, (float*)L.phi.p, st, prof ? ev + 4 : nullptr,
+    if ((rc = launch_fields(c, L, g, L.grid.p, (float*)L.phi.p, o.lines, st, prof ? ev + 4 : nullptr,
                             fork ? c->ev_join : nullptr)))
       return rc;
   } else {
@@ -954,7 +973,11 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
                                                                               prof ? ev + 4 : nullptr,
                                                                               fork ? c->ev_join : nullptr)))
       return rc;
-    k_diff64<<<(int)((g.ncell + 255) / 256), 256, 0, st>>>((const double*)L.phi.p, L.sc, (double*)L.E64.p);
+    const int nd = (int)((g.ncell + 255) / 256);
+    if (o.lines)
+      k_diff64<true><<<nd, 256, 0, st>>>((const double*)L.phi.p, L.sc, (double*)L.E64.p);
+    else
+      k_diff64<false><<<nd, 256, 0, st>>>((const double*)L.phi.p, L.sc, (double*)L.E64.p);
     LAUNCHCHK("k_diff64");
   }
   mark(9);
@@ -1098,7 +1121,7 @@ int apply_via_graph(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t 
   const bool reuse = o.sort && o.sort->order_in;
   auto& A = c->ag[reuse ? 1 : 0];
   const std::vector<int64_t> key = {(int64_t)(intptr_t)r, ld, (int64_t)(intptr_t)q, in.n, g.d.nx, g.d.ny, g.d.nz,
-                                    prec, o.sort != nullptr, reuse, o.sort && o.sort->order_out, c->rec_direct,
+                                    prec, o.sort != nullptr, o.lines, reuse, o.sort && o.sort->order_out, c->rec_direct,
                                     c->overlap,
                                     c->deposit_xcd, c->deposit_agg,
                                     c->deposit_tile, c->fft_plan, c->sort_cells, c->red_blocks, c->grid_clear,
@@ -1370,6 +1393,8 @@ int ocsc_apply_cells(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_
     sb.order_in = reuse ? (const uint32_t*)c->apply_order.p : nullptr;
     o.sort = &sb;
   }
+  o.lines = !o.sort && line_fields(L, g, n, prec);
+  if (!L.phi.p || (prec == OCSC_FP64 && !L.E64.p)) return fail(OCSC_ENOMEM, "field workspace");
   if (c->apply_graph && !cells && !c->profiling)
     rc = apply_via_graph(c, L, g, r, ld, q, in, prec, st, o);
   else
@@ -1547,7 +1572,7 @@ int ocsc_el_field(ocsc_ctx* c, const double* xyz, int64_t ld, const double* q, i
   } else {
     k_deposit_xyz<1><<<npart, kPT, 0, st>>>(R, q, L.sc, (unsigned long long*)L.grid.p);
     if ((rc = launch_kernel_spectrum<float>(c, L, g, st, 0))) return rc;
-    if ((rc = launch_fields(c, L, g, L.grid.p, (float*)L.phi.p, st))) return rc;
+    if ((rc = launch_fields(c, L, g, L.grid.p, (float*)L.phi.p, false, st))) return rc;
     k_gather_xyz<float><<<npart, kPT, 0, st>>>(R, (const float*)L.phi.p, L.sc, E, lde, cells);
   }
   LAUNCHCHK("el_field");

@@ -17,7 +17,7 @@
 // Fused multiply-adds appear only where numpy's BLAS call uses them (the 3x3
 // frame rotation, fma(x2,T2k, fma(x1,T1k, x0*T0k))).
 #pragma once
-#include "common.hpp"
+#include "mesh.hpp"
 
 namespace ocsc {
 
@@ -1204,6 +1204,83 @@ __device__ __forceinline__ void gather_field3(const float* __restrict__ E, const
   }
 }
 
+// Lower nodes of the two samplings of each axis, at X (0) and at X + 1/2 (1),
+// and whether they lie on the mesh.  Nodes are in [0, n - 2] in any case, and
+// those at X + 1/2 at most one above those at X.
+__device__ __forceinline__ void sample_nodes(const int* n, const double* X, int (*f)[3], bool (*ok)[3]) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double c = h ? X[k] + 0.5 : X[k];
+      ok[h][k] = c >= 0 && c <= n[k] - 1;
+      const double lo = c > 0 ? __builtin_floor(c) : 0.0;  // NaN: 0
+      f[h][k] = lo < n[k] - 2 ? (int)lo : n[k] - 2;
+    }
+}
+
+// gather_field3 from the field lines (FieldLine): all loads of a row hit the
+// line of the plane at X; offsets are 32-bit (at most 2 GB of fields).  The
+// same values and operations, so the same bits.
+__device__ __forceinline__ void gather_lines3(const float* __restrict__ E, const int* n, const double* X,
+                                              float* out) {
+  using L = FieldLine<float>;
+  int f[2][3];
+  float t[2][3];
+  bool ok[2][3];
+  sample_nodes(n, X, f, ok);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) t[h][k] = (float)((h ? X[k] + 0.5 : X[k]) - (double)f[h][k]);
+  const unsigned sy = (unsigned)(L::per_row(n[2]) * L::W), sx = (unsigned)n[1] * sy;
+  const unsigned zb = (unsigned)f[0][2] / L::KB, oz = zb * (L::W - L::KB);  // + z: word of the plane in its line
+  const char* base = (const char*)E;
+  // the loads first, row by row of the nodes: those that share a line follow
+  // each other
+  float2 pr[3][2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) {
+        const int i0 = f[ax == 0 ? 0 : 1][0], i1 = f[ax == 1 ? 0 : 1][1], i2 = f[ax == 2 ? 0 : 1][2];
+        const unsigned o = (unsigned)(i0 + a) * sx + (unsigned)(i1 + b) * sy + oz + (unsigned)i2 + ax * L::CW;
+        __builtin_memcpy(&pr[ax][a][b], base + (size_t)(o * 4u), sizeof(float2));
+      }
+#pragma unroll
+  for (int ax = 0; ax < 3; ++ax) {
+    const int h0 = ax == 0 ? 0 : 1, h1 = ax == 1 ? 0 : 1, h2 = ax == 2 ? 0 : 1;
+    const int i0 = f[h0][0], i1 = f[h1][1], i2 = f[h2][2];
+    float v[2][2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        bool z0 = false, z1 = false;  // corners on the component's last plane read 0
+        if (ax == 0) z0 = z1 = i0 + a >= n[0] - 1;
+        if (ax == 1) z0 = z1 = i1 + b >= n[1] - 1;
+        if (ax == 2) {
+          z0 = i2 >= n[2] - 1;
+          z1 = i2 + 1 >= n[2] - 1;
+        }
+        v[a][b][0] = z0 ? 0.f : pr[ax][a][b].x;
+        v[a][b][1] = z1 ? 0.f : pr[ax][a][b].y;
+      }
+  const float tx = t[h0][0], ty = t[h1][1], tz = t[h2][2];
+    float r[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const float q0 = __builtin_fmaf(tz, v[a][0][1] - v[a][0][0], v[a][0][0]);
+      const float q1 = __builtin_fmaf(tz, v[a][1][1] - v[a][1][0], v[a][1][0]);
+      r[a] = __builtin_fmaf(ty, q1 - q0, q0);
+    }
+    const float res = __builtin_fmaf(tx, r[1] - r[0], r[0]);
+    out[ax] = (ok[h0][0] && ok[h1][1] && ok[h2][2]) ? res : 0.f;
+  }
+}
+
 // field at a particle from the mesh result: FP64 potential (differenced
 // here, as the reference does) or, in the mixed form, three FP32 field grids
 // stored one after the other
@@ -1238,6 +1315,8 @@ __device__ __forceinline__ void gather_field(const F* __restrict__ phi, const Ki
 // from the potential, the arrays the reference interpolates (sc.py:198-204);
 // the kick then reads 8 corner values per component instead of 16 potential
 // values and divides nothing.  Stored one after the other, C order.
+// LINES: in the field layout (FieldLine).
+template <bool LINES = false>
 __device__ __forceinline__ void diff64_body(const double* __restrict__ phi, const KickScalars* __restrict__ scp,
                                             double* __restrict__ E, const int bx, const int nbx) {
   const int nx = scp->nmesh[0], ny = scp->nmesh[1], nz = scp->nmesh[2];
@@ -1247,14 +1326,22 @@ __device__ __forceinline__ void diff64_body(const double* __restrict__ phi, cons
   const int64_t sx = (int64_t)ny * nz;
   const int i = (int)(o / sx), j = (int)((o / nz) % ny), k = (int)(o % nz);
   const double p0 = phi[o];
-  E[o] = i < nx - 1 ? (p0 - phi[o + sx]) / scp->steps[0] : 0.0;
-  E[nc + o] = j < ny - 1 ? (p0 - phi[o + nz]) / scp->steps[1] : 0.0;
-  E[2 * nc + o] = k < nz - 1 ? (p0 - phi[o + 1]) / scp->steps[2] : 0.0;
+  const double e[3] = {i < nx - 1 ? (p0 - phi[o + sx]) / scp->steps[0] : 0.0,
+                       j < ny - 1 ? (p0 - phi[o + nz]) / scp->steps[1] : 0.0,
+                       k < nz - 1 ? (p0 - phi[o + 1]) / scp->steps[2] : 0.0};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if constexpr (LINES)
+      store_field(E, (int64_t)i * ny + j, k, nz, c, e[c]);
+    else
+      E[c * nc + o] = e[c];
+  }
 }
 
+template <bool LINES>
 __global__ void __launch_bounds__(256) k_diff64(const double* __restrict__ phi, const KickScalars* __restrict__ scp,
                                                 double* __restrict__ E) {
-  diff64_body(phi, scp, E, blockIdx.x, gridDim.x);
+  diff64_body<LINES>(phi, scp, E, blockIdx.x, gridDim.x);
 }
 
 // trilinear interpolation of a k_diff64 component, in gather_diff's order of
@@ -1304,6 +1391,50 @@ __device__ __forceinline__ void gather_field64(const double* __restrict__ E3, co
   E[2] = gather_grid64<2>(E3 + 2 * nc, nx, ny, nz, cz);
 }
 
+// gather_field64 from the field lines, each component in gather_grid64's order
+// of corners and operations (the same result bit for bit)
+__device__ __forceinline__ void gather_lines64(const double* __restrict__ E3, const KickScalars& s, const double* X,
+                                               double* E) {
+  using L = FieldLine<double>;
+  const int n[3] = {s.nmesh[0], s.nmesh[1], s.nmesh[2]};
+  int f[2][3];
+  bool ok[2][3];
+  sample_nodes(n, X, f, ok);
+  const unsigned sy = (unsigned)(L::per_row(n[2]) * L::W), sx = (unsigned)n[1] * sy;
+  const unsigned zb = (unsigned)f[0][2] / L::KB, oz = zb * (L::W - L::KB);  // + z: word of the plane in its line
+  double acc[3] = {0, 0, 0};
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int ax = 0; ax < 3; ++ax) {
+        const int h0 = ax == 0 ? 0 : 1, h1 = ax == 1 ? 0 : 1, h2 = ax == 2 ? 0 : 1;
+        const int i0 = f[h0][0], i1 = f[h1][1], i2 = f[h2][2];
+        const double t0 = (h0 ? X[0] + 0.5 : X[0]) - (double)i0, t1 = (h1 ? X[1] + 0.5 : X[1]) - (double)i1,
+                     t2 = (h2 ? X[2] + 0.5 : X[2]) - (double)i2;
+        // the two z-neighbours of a corner pair in one 16-byte load
+        double2 pr;
+        const unsigned o = (unsigned)(i0 + a) * sx + (unsigned)(i1 + b) * sy + oz + (unsigned)i2 + ax * L::CW;
+        __builtin_memcpy(&pr, E3 + o, sizeof(pr));
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const double ev = e ? pr.y : pr.x;
+          const double w = (a ? t0 : 1 - t0) * (b ? t1 : 1 - t1) * (e ? t2 : 1 - t2);
+          acc[ax] += w * ev;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int ax = 0; ax < 3; ++ax) {
+    const bool in = ok[ax == 0 ? 0 : 1][0] && ok[ax == 1 ? 0 : 1][1] && ok[ax == 2 ? 0 : 1][2];
+    E[ax] = in ? acc[ax] : 0.0;
+  }
+  E[0] = E[0] * s.gamma0;
+  E[1] = E[1] * s.gamma0;
+}
+
 // pass D: gather, kick in the rotated frame, rotate back, write all six rows
 // in place (sc.py:241-251, coord_transform.py:16-54).
 // Tracking fusions: DRIFT applies the next step's drift to the written rows
@@ -1321,7 +1452,8 @@ constexpr int kKickPT = 256;
 // deposit (the z pass that read them ran before this kick).
 // RECIN (with RECOUT): particle p is read from the record rec[perm[p]] that
 // it is written back to, instead of column p of r
-template <typename F, bool DRIFT, bool SUMP, bool RECOUT, bool RECIN = false>
+// LINES: phi holds the fields in the line layout (FieldLine)
+template <typename F, bool DRIFT, bool SUMP, bool RECOUT, bool RECIN = false, bool LINES = false>
 __device__ __forceinline__ void kick_body(double* __restrict__ r, int64_t ld, const F* __restrict__ phi,
                                           const KickScalars* __restrict__ scp, DriftArgs dr, double* __restrict__ part,
                                           const uint32_t* __restrict__ perm, PRec* __restrict__ rec,
@@ -1362,12 +1494,17 @@ __device__ __forceinline__ void kick_body(double* __restrict__ r, int64_t ld, co
     rot(xp + 3, s.T, pr);
     if constexpr (FAST) {
       float g[3];
-      gather_field3((const float*)phi, nn, X, g);
+      if constexpr (LINES)
+        gather_lines3((const float*)phi, nn, X, g);
+      else
+        gather_field3((const float*)phi, nn, X, g);
       E[0] = (double)g[0] * s.gamma0;
       E[1] = (double)g[1] * s.gamma0;
       E[2] = (double)g[2];
+    } else if constexpr (LINES) {
+      gather_lines64((const double*)phi, s, X, E);  // phi: the k_diff64 fields
     } else {
-      gather_field64((const double*)phi, s, X, E);  // phi: the k_diff64 fields
+      gather_field64((const double*)phi, s, X, E);
     }
     pr[0] = pr[0] + s.kperp * E[0];
     pr[1] = pr[1] + s.kperp * E[1];
@@ -1407,14 +1544,14 @@ __device__ __forceinline__ void kick_body(double* __restrict__ r, int64_t ld, co
   }
 }
 
-template <typename F, bool DRIFT = false, bool SUMP = false, bool RECOUT = false, bool RECIN = false>
+template <typename F, bool DRIFT = false, bool SUMP = false, bool RECOUT = false, bool RECIN = false, bool LINES = false>
 __global__ void __launch_bounds__(kKickPT) k_kick(double* __restrict__ r, int64_t ld, const F* __restrict__ phi,
                                                   const KickScalars* __restrict__ scp, DriftArgs dr = {0, 0},
                                                   double* __restrict__ part = nullptr,
                                                   const uint32_t* __restrict__ perm = nullptr,
                                                   PRec* __restrict__ rec = nullptr,
                                                   unsigned long long* __restrict__ zg = nullptr, int64_t zn = 0) {
-  kick_body<F, DRIFT, SUMP, RECOUT, RECIN>(r, ld, phi, scp, dr, part, perm, rec, zg, zn, blockIdx.x, gridDim.x);
+  kick_body<F, DRIFT, SUMP, RECOUT, RECIN, LINES>(r, ld, phi, scp, dr, part, perm, rec, zg, zn, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
