@@ -583,11 +583,11 @@ __device__ __forceinline__ void grid_add(unsigned long long* g, int64_t idx, lon
     atomicAdd(g + idx, (unsigned long long)v);
 }
 
-// NGP cell of a particle from its six rows, -1 if outside the mesh; FAST
-// (mixed form) takes the reciprocal-multiply transforms, the FP64 form the
-// exact sequence of the reference
+// NGP node (c[0], c[1], c[2]) of a particle from its six rows, false if outside
+// the mesh; FAST (mixed form) takes the reciprocal-multiply transforms, the
+// FP64 form the exact sequence of the reference
 template <bool FAST>
-__device__ __forceinline__ int64_t ngp_cell(const double* R6, const KickScalars& s) {
+__device__ __forceinline__ bool ngp_node(const double* R6, const KickScalars& s, int* c) {
   double xp[6], xyz[3], X[3];
   if constexpr (FAST)
     to_xp_fast(R6[0], R6[1], R6[2], R6[3], R6[4], R6[5], s, xp);
@@ -599,10 +599,20 @@ __device__ __forceinline__ int64_t ngp_cell(const double* R6, const KickScalars&
     grid_coords_fast(xyz, s, X);
   else
     grid_coords(xyz, s, X);
-  const int nx = s.nmesh[0], ny = s.nmesh[1], nz = s.nmesh[2];
   const double f0 = __builtin_floor(X[0]) + 1, f1 = __builtin_floor(X[1]) + 1, f2 = __builtin_floor(X[2]) + 1;
-  if (!(f0 >= 0 && f0 < nx && f1 >= 0 && f1 < ny && f2 >= 0 && f2 < nz)) return -1;
-  return ((int64_t)f0 * ny + (int64_t)f1) * nz + (int64_t)f2;
+  if (!(f0 >= 0 && f0 < s.nmesh[0] && f1 >= 0 && f1 < s.nmesh[1] && f2 >= 0 && f2 < s.nmesh[2])) return false;
+  c[0] = (int)f0;
+  c[1] = (int)f1;
+  c[2] = (int)f2;
+  return true;
+}
+
+// its flat cell index, -1 if outside the mesh
+template <bool FAST>
+__device__ __forceinline__ int64_t ngp_cell(const double* R6, const KickScalars& s) {
+  int c[3];
+  if (!ngp_node<FAST>(R6, s, c)) return -1;
+  return ((int64_t)c[0] * s.nmesh[1] + c[1]) * s.nmesh[2] + c[2];
 }
 
 // Deposit, pass C.  A workgroup handles kDepItems consecutive particles per
