@@ -295,8 +295,8 @@ struct ocsc_ctx {
   int sort_cells = 1;   // sort keys: bricks and the cells inside them (1), or bricks only (0)
   int sort_ahead = 1;   // tracking sort keys at the position half-way through the re-sort interval
   int resort_near = 0;  // re-sorts of the copy: one gather of rows, charges and permutation (1), or records
-  // charge grid cleared by a kernel on the side stream (1), by pass B (0), or
-  // in tracking by the previous step's kick (2; the first step as 1)
+  // charge grid cleared by pass B (0), on the second queue where that is faster
+  // (1), or in tracking by the previous step's kick (2; the first step as 1)
   int grid_clear = 1;
   // workgroups of the Green's-function node and difference kernels (grid-
   // stride loops; 0: one thread per node or cell): fewer leave more of the
@@ -755,6 +755,7 @@ struct StepOpts {
   // z pass, its last reader, runs before the kick)
   bool grid_zeroed = false;
   bool zero_next = false;
+  bool many = false;     // one of many launches of its loop (LSC kicks, moments)
   bool ordered = false;  // the rows are in cell order (the copy of a tracking call)
   bool lines = false;    // the fields in the line layout (FieldLine; buffers sized for it by the caller)
 };
@@ -848,11 +849,13 @@ int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // 177 -> 158, 1.5M / 63^3 403 -> 358, 4M / 127^3 mixed 873 -> 856.  One particle
 // per thread up to 150k (100k: 147 either way, 200k: 162 with one, 158 with
 // eight).  In cell order the table pays (2M / 63^3 FP64 tracking step 224 us
-// with it, 351 without), at two particles per thread (231 with eight).
+// with it, 351 without): the FP64 form at two particles per thread (231 with
+// eight), the mixed form at four (the first 20 steps of 10M / 127^3, whose order
+// decays fastest: 15.2 ms, 15.7 with two; later ones 14.1 with either).
 constexpr int64_t kDepOneMax = 150000;
-int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered) {
+int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered, int nword) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return 6;
+  if (ordered) return nword == 2 ? 6 : 1;
   return n <= kDepOneMax ? 5 : 3;
 }
 
@@ -861,7 +864,7 @@ template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
                     int32_t* cells, int64_t n, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = dep_tile(c, n, ordered);
+  const int t = dep_tile(c, n, ordered, NWORD);
   if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
   if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \
@@ -907,6 +910,11 @@ void launch_kick(ocsc_ctx* c, Lane& L, int npart, double* r, int64_t ld, const S
                                                       zg, zg ? nz64 : 0);
 }
 
+// cells from which the kernel spectrum is built on the second queue, and in a
+// loop with many other launches; bytes from which a captured clear is there
+constexpr int64_t kForkCells = 65536, kForkCellsMany = 524288;
+constexpr int64_t kSideClearBytes = 8 << 20;
+
 template <typename F, int NWORD>
 int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld, const double* q, const KickInputs& in,
                  int prec, hipStream_t st, const StepOpts& o = StepOpts()) {
@@ -928,16 +936,24 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // the kernel spectrum, which needs only the cell sizes, is built while the
   // deposit and the z and y passes run; the main stream waits for it only
   // before the x pass, its first reader.
-  const bool fork = c->overlap && !prof;
-  // the charge grid (all copies, all words): cleared by its own kernel on the
-  // side stream while the frame passes run, the deposit waiting for it on the
-  // second queue (option grid_clear 1), or by pass B (0; also when profiling
-  // or without the second stream).  10M / 127^3 mixed, 20-step calls on one
-  // GPU: 0.857 vs 0.870 ms per step (pass B's stores cost more than the
-  // cross-queue wait).  Tracking with grid_clear 2: the previous step's kick
-  // cleared it (o.grid_zeroed), no clear and no wait here.
+  // Not for small meshes, whose spectrum takes less time than the second
+  // queue's events: 20k / 31^3 FP64 kick 137 -> 115 us in line (115 -> 113 from
+  // a graph), 200k / 31^3 153 -> 144; 800k / 63^3 214 us beside the deposit, 226
+  // in line.  Launch by launch in a loop of many other launches (LSC, moments)
+  // the events are host time too: 800k / 63x63x95 377 us per step beside, 364 in
+  // line.
+  const bool capturing = st == c->cap_stream;
+  const bool fork = c->overlap && !prof && g.ncell >= (o.many && !capturing ? kForkCellsMany : kForkCells);
+  // The charge grid (all copies, all words) is cleared by pass B: its stores
+  // ride on the rows' reads, where a clear on the second queue costs two more
+  // events (one-shot kicks launch by launch 23 us less in pass B at every size,
+  // tracking steps 3 to 15 us).  With option grid_clear 1 a captured one-shot
+  // kick of a large grid keeps the second queue, whose edges cost less in a
+  // graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  Tracking with
+  // grid_clear 2: the previous step's kick cleared it (o.grid_zeroed).
   const int64_t nz64 = (c->deposit_xcd ? kNumXcd : 1) * NWORD * g.ncell;
-  const bool side_clear = c->grid_clear && fork && !o.grid_zeroed;
+  const bool side_clear =
+      c->grid_clear && fork && capturing && o.passA && !o.sump && !o.ordered && nz64 * 8 >= kSideClearBytes;
   unsigned long long* const zg = side_clear || o.grid_zeroed ? nullptr : (unsigned long long*)L.grid.p;
   if (side_clear) {
     HIPCHK(hipEventRecord(c->ev_fork0, st));
@@ -2182,6 +2198,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
     }
     o.dr = DriftArgs{Ld, r56};
     o.ordered = sorted;
+    o.many = tw || lq;
     o.grid_zeroed = c->grid_clear == 2 && step > 0;
     o.zero_next = c->grid_clear == 2 && step < nsteps - 1;
     if (ktime) {
