@@ -17,7 +17,7 @@
 // Every sum goes through fixed reduction trees: results do not depend on
 // launch timing.  The kernels after the statistics read one LscPlan, formed
 // either on the host (one-shot kicks: any grid size, one synchronisation) or
-// by k_lsc_plan on the device (kicks inside captured tracking graphs).
+// by the last statistics reduction on the device (kicks inside captured tracking graphs).
 #pragma once
 #include "particles.hpp"
 
@@ -41,14 +41,16 @@ constexpr int kLscKind[4] = {1, 0, 1, 0};
 
 template <int PASS>
 __global__ void __launch_bounds__(kPT) k_lsc_stat(Rows R, const double* __restrict__ q,
-                                                  const LscState* __restrict__ sp, double* __restrict__ part) {
+                                                  const LscState* __restrict__ sp, double* __restrict__ part,
+                                                  int64_t n) {
   constexpr int NV = kLscNV[PASS], KIND = kLscKind[PASS];
   __shared__ double lds[(kPT / 64) * NV];
-  const LscState s = *sp;
+  LscState s{};
+  if constexpr (PASS != 0) s = *sp;  // pass 0 runs before the state is set up (by its reduction)
   double acc[NV];
 #pragma unroll
   for (int c = 0; c < NV; ++c) acc[c] = (KIND == 1 && c < 3) ? __builtin_inf() : ((KIND == 1 && c < 6) ? -__builtin_inf() : 0.0);
-  for (int64_t i = (int64_t)blockIdx.x * kPT + threadIdx.x; i < s.n; i += (int64_t)gridDim.x * kPT) {
+  for (int64_t i = (int64_t)blockIdx.x * kPT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kPT) {
     const double tau = R.r[4 * R.ld + i];
     if constexpr (PASS == 0) {
       acc[0] = tau < acc[0] ? tau : acc[0];
@@ -80,39 +82,6 @@ __global__ void __launch_bounds__(kPT) k_lsc_stat(Rows R, const double* __restri
   block_reduce<NV, KIND>(acc, lds);
   if (threadIdx.x == 0)
     for (int c = 0; c < NV; ++c) part[c * gridDim.x + blockIdx.x] = acc[c];
-}
-
-template <int PASS>
-__global__ void __launch_bounds__(1024) k_lsc_stat_reduce(LscState* __restrict__ sp, const double* __restrict__ part,
-                                                          int nblk) {
-#pragma clang fp contract(off)
-  constexpr int NV = kLscNV[PASS], KIND = kLscKind[PASS];
-  __shared__ double lds[16 * NV];
-  double t[NV];
-  reduce_partials<NV, KIND>(part, nblk, t, lds);
-  if (threadIdx.x != 0) return;
-  LscState& s = *sp;
-  if constexpr (PASS == 0) {
-    s.tau_min = t[0];
-    s.tau_max = t[3];
-    s.tau_mean = t[6] / (double)s.n;
-    s.sumq = t[7];
-  } else if constexpr (PASS == 1) {
-    s.tau_std = __builtin_sqrt(t[0] / (double)s.n);
-    s.lo = s.tau_mean + s.tau_std * s.b0;
-    s.hi = s.tau_mean + s.tau_std * s.b1;
-  } else if constexpr (PASS == 2) {
-    s.xmin = t[0];
-    s.ymin = t[1];
-    s.xmax = t[3];
-    s.ymax = t[4];
-    s.cnt = t[6];
-    s.xmean = t[7] / t[6];
-    s.ymean = t[8] / t[6];
-  } else {
-    s.xvar = t[0] / s.cnt;
-    s.yvar = t[1] / s.cnt;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -530,14 +499,19 @@ __global__ void __launch_bounds__(1024) k_lsc_profile(const long long* __restric
   const int nbins = p->nbins, K = p->K;
   if (nbins == 0) return;
   const double ds = p->ds, sigma = p->sig;
-  if (threadIdx.x == 0) {
+  // one tap per thread; every one of them adds the taps up in their order
+  // (one thread taking 25 exponentials one after the other was half the time
+  // of this single-workgroup kernel)
+  __shared__ double E[kLscMaxTaps];
+  if ((int)threadIdx.x <= 2 * K) {
+    const double x = (double)((int)threadIdx.x - K) * ds / sigma;
+    E[threadIdx.x] = exp(-0.5 * (x * x));
+  }
+  __syncthreads();
+  if ((int)threadIdx.x <= 2 * K) {
     double gs = 0;
-    for (int m = 0; m <= 2 * K; ++m) {
-      const double x = (double)(m - K) * ds / sigma;
-      G[m] = exp(-0.5 * (x * x));
-      gs += G[m];
-    }
-    for (int m = 0; m <= 2 * K; ++m) G[m] = G[m] / gs;
+    for (int m = 0; m <= 2 * K; ++m) gs += E[m];
+    G[threadIdx.x] = E[threadIdx.x] / gs;
   }
   __syncthreads();
   double part = 0;
@@ -563,29 +537,63 @@ __global__ void __launch_bounds__(1024) k_lsc_profile(const long long* __restric
 }
 
 // ---------------------------------------------------------------------------
-// Inside tracking graphs: state set-up and the plan on the device (the
-// histogram on the plan's grid is moments.hpp k_cic_grid).
-__global__ void k_lsc_init(LscState* __restrict__ s, int64_t n, double b0, double b1) {
-  if (threadIdx.x != 0) return;
-  LscState h{};
-  h.n = n;
-  h.b0 = b0;
-  h.b1 = b1;
-  *s = h;
-}
+// Totals of a statistics pass, one workgroup.  Pass 0's sets the state up and
+// the last pass's (p given) forms the plan on the device (the histogram on the
+// plan's grid is moments.hpp k_cic_grid): a kick needs no launch for either.
+struct LscInit {
+  int64_t n;
+  double b0, b1;
+};
 
-__global__ void k_lsc_plan(const LscState* __restrict__ s, LscConst k, LscPlan* __restrict__ p, int* __restrict__ err) {
+template <int PASS>
+__global__ void __launch_bounds__(1024) k_lsc_stat_reduce(LscState* __restrict__ sp, const double* __restrict__ part,
+                                                          int nblk, LscInit in, LscConst k, LscPlan* __restrict__ p,
+                                                          int* __restrict__ err) {
+#pragma clang fp contract(off)
+  constexpr int NV = kLscNV[PASS], KIND = kLscKind[PASS];
+  __shared__ double lds[16 * NV];
+  double t[NV];
+  reduce_partials<NV, KIND>(part, nblk, t, lds);
   if (threadIdx.x != 0) return;
-  LscPlan q;
-  lsc_make_plan(*s, k, &q);
-  if (k.factors) {
-    const int i = *k.fctr;
-    if (i < k.nfactors) q.imp.factor = k.factors[i];
-    *k.fctr = i + 1;
+  LscState& s = *sp;
+  if constexpr (PASS == 0) {
+    LscState h{};
+    h.n = in.n;
+    h.b0 = in.b0;
+    h.b1 = in.b1;
+    s = h;
+    s.tau_min = t[0];
+    s.tau_max = t[3];
+    s.tau_mean = t[6] / (double)s.n;
+    s.sumq = t[7];
+  } else if constexpr (PASS == 1) {
+    s.tau_std = __builtin_sqrt(t[0] / (double)s.n);
+    s.lo = s.tau_mean + s.tau_std * s.b0;
+    s.hi = s.tau_mean + s.tau_std * s.b1;
+  } else if constexpr (PASS == 2) {
+    s.xmin = t[0];
+    s.ymin = t[1];
+    s.xmax = t[3];
+    s.ymax = t[4];
+    s.cnt = t[6];
+    s.xmean = t[7] / t[6];
+    s.ymean = t[8] / t[6];
+  } else {
+    s.xvar = t[0] / s.cnt;
+    s.yvar = t[1] / s.cnt;
   }
-  *p = q;
-  if (q.err && *err == 0) *err = q.err;
+  if constexpr (PASS >= 2) {
+    if (!p) return;  // pass 3 follows
+    LscPlan q;
+    lsc_make_plan(s, k, &q);
+    if (k.factors) {
+      const int i = *k.fctr;
+      if (i < k.nfactors) q.imp.factor = k.factors[i];
+      *k.fctr = i + 1;
+    }
+    *p = q;
+    if (q.err && *err == 0) *err = q.err;
+  }
 }
-
 
 }  // namespace ocsc

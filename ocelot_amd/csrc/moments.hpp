@@ -58,14 +58,17 @@ __device__ __forceinline__ void mom_corrected(const double* R6, const MomState& 
 // drift is applied to the rows after their moments are added, to every
 // particle (selected or not), with the drift kernel's fused multiply-adds:
 // x += L x', y += L y', tau += r56 delta.  rw is R.r, writable.
+// The first pass (0 or 6) takes the working state as an argument, and its
+// reduction writes it: no launch or copy to set it up.
 template <int PASS, bool DRIFT = false>
 __global__ void __launch_bounds__(kPT) k_mom(Rows R, const double* __restrict__ q, const MomState* __restrict__ msp,
                                              double* __restrict__ part, double* rw = nullptr, double L = 0,
-                                             double r56 = 0) {
+                                             double r56 = 0, MomState s0 = MomState{}) {
   static_assert(!DRIFT || PASS == 5, "the drift rides on the last pass");
+  constexpr bool kFirst = PASS == 0 || PASS == 6;
   constexpr int NV = kMomNV[PASS];
   __shared__ double lds[(kPT / 64) * NV];
-  const MomState s = *msp;
+  const MomState s = kFirst ? s0 : *msp;
   double acc[NV];
 #pragma unroll
   for (int c = 0; c < NV; ++c) acc[c] = 0;
@@ -166,16 +169,21 @@ __global__ void __launch_bounds__(kPT) k_mom(Rows R, const double* __restrict__ 
     for (int c = 0; c < NV; ++c) part[c * gridDim.x + blockIdx.x] = acc[c];
 }
 
-// one block: totals of a pass, then the scalars the next pass needs
+// one block: totals of a pass, then the scalars the next pass needs.  After
+// the last pass the state is appended to the step table of a tracking call
+// (table, or null) at a device-side counter.
 template <int PASS>
 __global__ void __launch_bounds__(1024) k_mom_reduce(MomState* __restrict__ msp, const double* __restrict__ part,
-                                                     int nblk) {
+                                                     int nblk, MomState s0 = MomState{},
+                                                     MomState* __restrict__ table = nullptr,
+                                                     int* __restrict__ counter = nullptr, int cap = 0) {
   constexpr int NV = kMomNV[PASS];
   __shared__ double lds[16 * NV];
   double t[NV];
   reduce_partials<NV, 0>(part, nblk, t, lds);
   if (threadIdx.x != 0) return;
   MomState& s = *msp;
+  if constexpr (PASS == 0 || PASS == 6) s = s0;
   const double n = (double)s.n;
   if constexpr (PASS == 0) {
     s.tau_all = t[0] / n;
@@ -204,36 +212,12 @@ __global__ void __launch_bounds__(1024) k_mom_reduce(MomState* __restrict__ msp,
     for (int k = 0; k < 4; ++k) s.c[k] = t[k] / s.cnt;
   } else {
     for (int k = 0; k < 12; ++k) s.mom[k] = t[k] / s.cnt;
+    if (table) {
+      const int k = *counter;
+      if (k < cap) table[k] = s;
+      *counter = k + 1;
+    }
   }
-}
-
-// Per-step moments inside a tracking loop (graph-capturable: no host copies).
-// k_mom_init fills the working state from scalars; k_mom_store appends it to
-// the step table at a device-side counter.
-__global__ void k_mom_init(MomState* __restrict__ s, int64_t n, int bounds, int disp_mode, double b0, double b1,
-                           double d0, double d1, double d2, double d3) {
-  if (threadIdx.x != 0) return;
-  MomState m{};
-  m.n = n;
-  m.bounds = bounds;
-  m.disp_mode = disp_mode;
-  m.b0 = b0;
-  m.b1 = b1;
-  if (disp_mode == 1) {
-    m.D[0] = d0;
-    m.D[1] = d1;
-    m.D[2] = d2;
-    m.D[3] = d3;
-  }
-  *s = m;
-}
-
-__global__ void k_mom_store(const MomState* __restrict__ s, MomState* __restrict__ table, int* __restrict__ counter,
-                            int cap) {
-  if (threadIdx.x != 0) return;
-  const int k = *counter;
-  if (k < cap) table[k] = *s;
-  *counter = k + 1;
 }
 
 __global__ void k_counter_reset(int* __restrict__ counter) {
@@ -307,29 +291,39 @@ __global__ void __launch_bounds__(kPT) k_cic(Rows R, int64_t n, double a, double
   for (int j = threadIdx.x; j < nb; j += kPT) hist[(int64_t)blockIdx.x * nb + j] = h[j];
 }
 
-// Totals of the per-workgroup histograms: a workgroup takes 64 bins, its 16
-// waves add every 16th histogram, then wave 0 adds the 16 wave sums.  The
-// sums are integers, so the result is exact in any order.  nbins_dev, when
-// given, overrides nbins (a grid planned on the device); workgroups beyond
-// the bins return at once.
+// Totals of the per-workgroup histograms: a workgroup takes kCicSumBins bins
+// (one 128-byte line of every histogram), 64 threads per bin.  With 64 bins
+// and 16 threads per bin the few hundred bins of a profile left all but a
+// handful of CUs idle (20.7 us for 1024 histograms of 350 bins).  The sums are
+// integers, so the result is exact in any order.  nbins_dev, when given,
+// overrides nbins (a grid planned on the device); workgroups beyond the bins
+// return at once.
 constexpr int kCicBlocks = 1024;  // workgroups of the histogram pass
+constexpr int kCicSumBins = 16;
 
 __global__ void __launch_bounds__(1024) k_cic_sum(const long long* __restrict__ hist, int nblk, int nbins,
                                                   const int* __restrict__ nbins_dev, long long* __restrict__ out) {
-  __shared__ long long part[16][64];
+  __shared__ long long part[16][kCicSumBins];
   const int nb = nbins_dev ? *nbins_dev : nbins;
-  if ((int)blockIdx.x * 64 >= nb) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int j = blockIdx.x * 64 + lane;
+  if ((int)blockIdx.x * kCicSumBins >= nb) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, bin = lane & (kCicSumBins - 1);
+  const int j = blockIdx.x * kCicSumBins + bin;
   long long acc = 0;
-  if (j < nb)
-    for (int b = w; b < nblk; b += 16) acc += hist[(int64_t)b * nb + j];
-  part[w][lane] = acc;
+  if (j < nb) {
+#pragma unroll 16
+    for (int b = threadIdx.x / kCicSumBins; b < nblk; b += 1024 / kCicSumBins) acc += hist[(int64_t)b * nb + j];
+  }
+  acc += __shfl_xor(acc, 16);
+  acc += __shfl_xor(acc, 32);
+  if (lane < kCicSumBins) part[w][lane] = acc;
   __syncthreads();
-  if (w == 0 && j < nb) {
+  if (w == 0) {
     long long t = 0;
-    for (int k = 0; k < 16; ++k) t += part[k][lane];
-    out[j] = t;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t += part[4 * (lane / kCicSumBins) + k][bin];
+    t += __shfl_xor(t, 16);
+    t += __shfl_xor(t, 32);
+    if (lane < kCicSumBins && j < nb) out[j] = t;
   }
 }
 

@@ -1760,10 +1760,23 @@ int cic_profile(Buf& buf, const Rows& R, int64_t n, double a, double ds, int nbi
   for (int j0 = 0; j0 < nbins; j0 += win) {
     const int nb = std::min(win, nbins - j0);
     k_cic<<<ncic, kPT, (size_t)nb * sizeof(long long), st>>>(R, n, a, ds, nbins, j0, nb, wscale, hist);
-    k_cic_sum<<<(nb + 63) / 64, 1024, 0, st>>>(hist, ncic, nb, nullptr, *tot + j0);
+    k_cic_sum<<<(nb + kCicSumBins - 1) / kCicSumBins, 1024, 0, st>>>(hist, ncic, nb, nullptr, *tot + j0);
   }
   LAUNCHCHK("k_cic");
   return OCSC_OK;
+}
+
+// working state before the first pass of the moments
+MomState mom_start(int64_t n, int bounds, int disp_mode, double b0, double b1, const double* disp) {
+  MomState m{};
+  m.n = n;
+  m.bounds = bounds;
+  m.disp_mode = disp_mode;
+  m.b0 = b0;
+  m.b1 = b1;
+  if (disp_mode == 1)
+    for (int k = 0; k < 4; ++k) m.D[k] = disp[k];
+  return m;
 }
 
 // Centre of the peak-current window (analysis.py:61-64): the current profile
@@ -1850,28 +1863,19 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
   const int nblk = nred_blocks(c, n);
   int rc;
   if ((rc = ensure(L.part, (size_t)12 * nblk * sizeof(double)))) return rc;
-  // the pinned mirror may still be read by an earlier copy on another stream
-  HIPCHK(hipStreamSynchronize(st));
-  MomState& h = *c->mom_host;
-  std::memset(&h, 0, sizeof(h));
-  h.n = n;
-  h.bounds = (flags & OCSC_MOM_BOUNDS) ? 1 : 0;
-  h.b0 = b0;
-  h.b1 = b1;
-  h.disp_mode = (flags & OCSC_MOM_DISP_GIVEN) ? 1 : ((flags & OCSC_MOM_AUTO_DISP) ? 2 : 0);
-  if (h.disp_mode == 1)
-    for (int k = 0; k < 4; ++k) h.D[k] = disp[k];
-  HIPCHK(hipMemcpyAsync(c->mom, &h, sizeof(h), hipMemcpyHostToDevice, st));
+  MomState& h = *c->mom_host;  // read back at the end (every call waits for its copies)
+  const MomState s0 = mom_start(n, (flags & OCSC_MOM_BOUNDS) ? 1 : 0,
+                                (flags & OCSC_MOM_DISP_GIVEN) ? 1 : ((flags & OCSC_MOM_AUTO_DISP) ? 2 : 0), b0, b1, disp);
   double* part = (double*)L.part.p;
   const Rows R{r, ld};
   double z0 = 0;
-  if (!h.bounds && h.disp_mode != 2) {
-    k_mom<6><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);  // passes 0, 2, 4 in one read
-    k_mom_reduce<6><<<1, 1024, 0, st>>>(c->mom, part, nblk);
+  if (!s0.bounds && s0.disp_mode != 2) {
+    k_mom<6><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, nullptr, 0.0, 0.0, s0);  // passes 0, 2, 4 in one read
+    k_mom_reduce<6><<<1, 1024, 0, st>>>(c->mom, part, nblk, s0);
   } else {
-    k_mom<0><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
-    k_mom_reduce<0><<<1, 1024, 0, st>>>(c->mom, part, nblk);
-    if (h.bounds) {
+    k_mom<0><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, nullptr, 0.0, 0.0, s0);
+    k_mom_reduce<0><<<1, 1024, 0, st>>>(c->mom, part, nblk, s0);
+    if (s0.bounds) {
       k_mom<1><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
       k_mom_reduce<1><<<1, 1024, 0, st>>>(c->mom, part, nblk);
       if (flags & OCSC_MOM_IMAX) {
@@ -1880,7 +1884,7 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
         z0 = -1;  // mean(tau), set below from the device state
       }
     }
-    if (h.disp_mode != 2) {
+    if (s0.disp_mode != 2) {
       k_mom<7><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);  // passes 2 and 4 in one read
       k_mom_reduce<7><<<1, 1024, 0, st>>>(c->mom, part, nblk);
     } else {
@@ -1907,7 +1911,7 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
   for (int k = 0; k < 12; ++k) v[12 + k] = h.mom[k];
   v[24] = h.tau_all;
   v[25] = h.std_all;
-  v[26] = (flags & OCSC_MOM_IMAX) && h.bounds ? z0 : h.tau_all;
+  v[26] = (flags & OCSC_MOM_IMAX) && s0.bounds ? z0 : h.tau_all;
   for (int k = 0; k < nout && k < OCSC_MOM_NOUT; ++k) out[k] = v[k];
   return OCSC_OK;
 }
@@ -1937,15 +1941,14 @@ int enqueue_moments(ocsc_ctx* c, const Rows& R, const double* q, int64_t n, cons
   const int nblk = nred_blocks(c, n);
   double* part = (double*)c->mom_part.p;
   MomState* cur = c->mom;
-  k_mom_init<<<1, 64, 0, st>>>(cur, n, t.bounds, t.disp_mode, t.b0, t.b1, t.disp[0], t.disp[1], t.disp[2],
-                               t.disp[3]);
+  const MomState s0 = mom_start(n, t.bounds, t.disp_mode, t.b0, t.b1, t.disp);
   const bool one_read = !t.bounds && t.disp_mode != 2;  // passes 0, 2, 4 together
   if (one_read) {
-    k_mom<6><<<nblk, kPT, 0, st>>>(R, q, cur, part);
-    k_mom_reduce<6><<<1, 1024, 0, st>>>(cur, part, nblk);
+    k_mom<6><<<nblk, kPT, 0, st>>>(R, q, cur, part, nullptr, 0.0, 0.0, s0);
+    k_mom_reduce<6><<<1, 1024, 0, st>>>(cur, part, nblk, s0);
   } else {
-    k_mom<0><<<nblk, kPT, 0, st>>>(R, q, cur, part);
-    k_mom_reduce<0><<<1, 1024, 0, st>>>(cur, part, nblk);
+    k_mom<0><<<nblk, kPT, 0, st>>>(R, q, cur, part, nullptr, 0.0, 0.0, s0);
+    k_mom_reduce<0><<<1, 1024, 0, st>>>(cur, part, nblk, s0);
   }
   if (t.bounds) {
     k_mom<1><<<nblk, kPT, 0, st>>>(R, q, cur, part);
@@ -1960,7 +1963,7 @@ int enqueue_moments(ocsc_ctx* c, const Rows& R, const double* q, int64_t n, cons
       k_imax_plan<<<1, 64, 0, st>>>(cur, c->imax_plan, cap, c->imax_err);
       k_cic_grid<ImaxPlan><<<kCicBlocks, kPT, (size_t)cap * sizeof(long long), st>>>(R, n, c->imax_plan,
                                                                                      cic_wscale(n), hist);
-      k_cic_sum<<<(cap + 63) / 64, 1024, 0, st>>>(hist, kCicBlocks, cap, &c->imax_plan->nbins, tot);
+      k_cic_sum<<<(cap + kCicSumBins - 1) / kCicSumBins, 1024, 0, st>>>(hist, kCicBlocks, cap, &c->imax_plan->nbins, tot);
       k_imax_peak<<<1, 1024, 0, st>>>(tot, c->imax_plan, cur);
     }
   }
@@ -1979,8 +1982,7 @@ int enqueue_moments(ocsc_ctx* c, const Rows& R, const double* q, int64_t n, cons
     k_mom<5, true><<<nblk, kPT, 0, st>>>(R, q, cur, part, const_cast<double*>(R.r), dr->L, dr->r56);
   else
     k_mom<5><<<nblk, kPT, 0, st>>>(R, q, cur, part);
-  k_mom_reduce<5><<<1, 1024, 0, st>>>(cur, part, nblk);
-  k_mom_store<<<1, 64, 0, st>>>(cur, (MomState*)c->mom_tab.p, (int*)c->mom_ctr.p, t.cap);
+  k_mom_reduce<5><<<1, 1024, 0, st>>>(cur, part, nblk, s0, (MomState*)c->mom_tab.p, (int*)c->mom_ctr.p, t.cap);
   LAUNCHCHK("tracking moments");
   return OCSC_OK;
 }
@@ -3510,18 +3512,21 @@ int lsc_buffers(ocsc_ctx* c, int64_t bins) {
 
 // slice statistics (sc.py:566-577) into c->lsc; the state is initialised by
 // the caller
-void lsc_stats(ocsc_ctx* c, const Rows& R, const double* q, int64_t n, int step_profile, hipStream_t st) {
+void lsc_stats(ocsc_ctx* c, const Rows& R, const double* q, int64_t n, const LscConst& k, double b0, double b1,
+               hipStream_t st) {
   double* part = (double*)c->lane0.part.p;
   const int nblk = nred_blocks(c, n);
-  k_lsc_stat<0><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part);
-  k_lsc_stat_reduce<0><<<1, 1024, 0, st>>>(c->lsc, part, nblk);
-  k_lsc_stat<1><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part);
-  k_lsc_stat_reduce<1><<<1, 1024, 0, st>>>(c->lsc, part, nblk);
-  k_lsc_stat<2><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part);
-  k_lsc_stat_reduce<2><<<1, 1024, 0, st>>>(c->lsc, part, nblk);
-  if (!step_profile) {
-    k_lsc_stat<3><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part);
-    k_lsc_stat_reduce<3><<<1, 1024, 0, st>>>(c->lsc, part, nblk);
+  const LscInit in{n, b0, b1};
+  LscPlan* const plan = c->lsc_plan;
+  k_lsc_stat<0><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part, n);
+  k_lsc_stat_reduce<0><<<1, 1024, 0, st>>>(c->lsc, part, nblk, in, k, nullptr, c->lsc_err);
+  k_lsc_stat<1><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part, n);
+  k_lsc_stat_reduce<1><<<1, 1024, 0, st>>>(c->lsc, part, nblk, in, k, nullptr, c->lsc_err);
+  k_lsc_stat<2><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part, n);
+  k_lsc_stat_reduce<2><<<1, 1024, 0, st>>>(c->lsc, part, nblk, in, k, k.step_profile ? plan : nullptr, c->lsc_err);
+  if (!k.step_profile) {
+    k_lsc_stat<3><<<nblk, kPT, 0, st>>>(R, q, c->lsc, part, n);
+    k_lsc_stat_reduce<3><<<1, 1024, 0, st>>>(c->lsc, part, nblk, in, k, plan, c->lsc_err);
   }
 }
 
@@ -3563,14 +3568,12 @@ int enqueue_lsc(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, 
                 double b1, hipStream_t st, const DriftArgs* dr, const LscSump* sm) {
   const int cap = k.cap;
   const int ncic = kCicBlocks;
-  k_lsc_init<<<1, 64, 0, st>>>(c->lsc, n, b0, b1);
-  lsc_stats(c, Rows{r, ld}, q, n, k.step_profile, st);
-  k_lsc_plan<<<1, 64, 0, st>>>(c->lsc, k, c->lsc_plan, c->lsc_err);
+  lsc_stats(c, Rows{r, ld}, q, n, k, b0, b1, st);
   long long* hist = (long long*)c->lsc_cic.p;
   long long* tot = hist + (size_t)ncic * cap;
   k_cic_grid<LscPlan><<<ncic, kPT, (size_t)cap * sizeof(long long), st>>>(Rows{r, ld}, n, c->lsc_plan, cic_wscale(n),
                                                                          hist);
-  k_cic_sum<<<(cap + 63) / 64, 1024, 0, st>>>(hist, ncic, cap, &c->lsc_plan->nbins, tot);
+  k_cic_sum<<<(cap + kCicSumBins - 1) / kCicSumBins, 1024, 0, st>>>(hist, ncic, cap, &c->lsc_plan->nbins, tot);
   LAUNCHCHK("k_cic_grid");
   return lsc_from_profile(c, r, ld, n, tot, cap, st, dr, sm);
 }
@@ -3606,7 +3609,6 @@ int ocsc_lsc_apply(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t 
   // in the middle); a profile that needs more bins than that path holds is
   // planned again on the host from the same statistics (the bunch is not
   // kicked by a refused plan)
-  k_counter_reset<<<1, 64, 0, st>>>(c->lsc_err);
   if ((rc = enqueue_lsc(c, r, ld, q, n,
                         lsc_const(step_profile, smooth_param, E_GeV, dz, K_max, fill_factor, kLscGraphBins), b0, b1,
                         st)))
