@@ -149,6 +149,60 @@ class Context:
         self.handle = h
         self.device = int(device)
         self.lock = threading.RLock()
+        self._stage = None       # pinned buffer of the host copies (at most STAGE_BYTES)
+        self._stage_free = None  # event: the buffer's last transfer has ended
+
+    # Copies between the GPU and a caller's ndarrays go through one pinned
+    # buffer, a chunk at a time.  The runtime's own path for pageable memory
+    # took 280 us up and 581 us down for the 9.6 MB of 200k particles (72 us for
+    # their charges), pinned memory 177 and 180 us, and the copy between the
+    # ndarray and the buffer, by all threads, 18 us.  Called with ``lock`` held.
+    STAGE_BYTES = 32 << 20
+
+    def _staging(self, nbytes):
+        import torch
+        if self._stage_free is not None:
+            self._stage_free.synchronize()  # a call that failed may have left a transfer running
+        want = min(int(nbytes), self.STAGE_BYTES)
+        if self._stage is None or self._stage.numel() * 8 < want:
+            self._stage = torch.empty((want + 7) // 8, dtype=torch.float64, pin_memory=True)
+            self._stage_free = torch.cuda.Event()
+        return self._stage
+
+    def upload(self, parts):
+        """float64 host tensors (contiguous) as one flat GPU tensor, on the
+        current stream of the device."""
+        import torch
+        total = sum(t.numel() for t in parts)
+        dst = torch.empty(total, dtype=torch.float64, device=f"cuda:{self.device}")
+        buf = self._staging(total * 8)
+        cap, at, fill = buf.numel(), 0, 0
+        for i, t in enumerate(parts):
+            flat, off = t.reshape(-1), 0
+            while off < flat.numel():
+                if fill == cap:
+                    dst[at:at + fill].copy_(buf[:fill], non_blocking=True)
+                    self._stage_free.record()
+                    self._stage_free.synchronize()
+                    at, fill = at + fill, 0
+                m = min(cap - fill, flat.numel() - off)
+                buf[fill:fill + m].copy_(flat[off:off + m])
+                off, fill = off + m, fill + m
+        if fill:
+            dst[at:at + fill].copy_(buf[:fill], non_blocking=True)
+            self._stage_free.record()
+        return dst
+
+    def download(self, src, host):
+        """A flat float64 GPU tensor into a contiguous host tensor."""
+        flat = host.reshape(-1)
+        buf = self._staging(flat.numel() * 8)
+        for off in range(0, flat.numel(), buf.numel()):
+            m = min(buf.numel(), flat.numel() - off)
+            buf[:m].copy_(src[off:off + m], non_blocking=True)
+            self._stage_free.record()
+            self._stage_free.synchronize()
+            flat[off:off + m].copy_(buf[:m])
 
     def __del__(self):
         try:

@@ -139,21 +139,22 @@ def _kick(proc, p_array, zstep, want_cells):
         return cells
     dev = _device_of(proc)
     # a C-ordered, writable float64 ndarray is copied to and from the GPU
-    # as it lies (no host-side temporaries); anything else goes through a
-    # contiguous copy and is assigned back element-wise
+    # as it lies (through the context's pinned buffer); anything else goes
+    # through a contiguous copy and is assigned back element-wise
     direct = _host_direct(r)
     with torch.cuda.device(dev), _lib.using(dev) as h:
         host = torch.from_numpy(r if direct else np.ascontiguousarray(r, dtype=np.float64))
-        rt = host.to(f"cuda:{dev}")
-        qt = torch.from_numpy(np.ascontiguousarray(p_array.q_array, dtype=np.float64)).to(f"cuda:{dev}")
+        ctx = _lib.context(dev)
+        both = ctx.upload((host, torch.from_numpy(np.ascontiguousarray(p_array.q_array, dtype=np.float64))))
+        rt, qt = both[:6 * n], both[6 * n:]
         cells = torch.empty(n, dtype=torch.int32, device=rt.device) if want_cells else None
         stream = torch.cuda.current_stream(dev).cuda_stream
         _lib.check(lib.ocsc_apply_cells(h, rt.data_ptr(), n, qt.data_ptr(), n, nmesh, E, float(zstep), rm, scale,
                                         shift, prec, 1, cells.data_ptr() if cells is not None else None, stream))
         if direct:
-            host.copy_(rt)
+            ctx.download(rt, host)
         else:
-            r[...] = rt.cpu().numpy()
+            r[...] = rt.reshape(6, n).cpu().numpy()
     return cells.cpu().numpy() if cells is not None else None
 
 
