@@ -63,21 +63,21 @@ __device__ __forceinline__ void seg_find(const BSeg& g, int& job, int& bx, int& 
   int lo = 0, hi = g.nj;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (g.pre[mid] <= b)
+    if (uniform_load(g.pre + mid) <= b)
       lo = mid;
     else
       hi = mid;
   }
-  job = g.ids[lo];
-  bx = (int)(b - g.pre[lo]);
-  nbx = (int)g.cnt[lo];
+  job = uniform_load(g.ids + lo);
+  bx = (int)(b - uniform_load(g.pre + lo));
+  nbx = (int)uniform_load(g.cnt + lo);
 }
 
 #define OCSC_BJOB()          \
   int j_, bx, nbx;           \
   seg_find(g, j_, bx, nbx);  \
   if (bx >= nbx) return;     \
-  const BJob& b = J[j_]
+  const BJob b = uniform_load(J + j_)
 
 __global__ void __launch_bounds__(kPT) kb_passA(const BJob* __restrict__ J, BSeg g) {
   OCSC_BJOB();

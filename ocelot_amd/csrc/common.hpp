@@ -104,6 +104,28 @@ struct KickScalars {
   double q_val;
 };
 
+// *p for a p that is the same in the whole workgroup, through the scalar cache
+// into scalar registers.  What a kernel reads through a pointer that it loaded
+// itself (the jobs of a batch and their scalars) the compiler loads per lane:
+// the batched kick took 112 vector registers that way, the single one 59.  For
+// data that this kernel does not write (the error words aside, which are read
+// at its start).
+template <class T>
+__device__ __forceinline__ T uniform_load(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
+  const uint64_t a = (uint64_t)p;
+  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32 |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+  const ConstWords c = (ConstWords)u;
+  uint32_t w[sizeof(T) / 4];
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 4; ++i) w[i] = c[i];
+  T t;
+  __builtin_memcpy(&t, w, sizeof(T));
+  return t;
+}
+
 enum ErrBits : int32_t { kErrNonFinite = 1, kErrZeroCharge = 2, kErrCell = 4, kErrSteps = 8 };
 
 __host__ __device__ constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v >> 1); }

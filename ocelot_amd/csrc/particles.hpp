@@ -359,7 +359,7 @@ __device__ __forceinline__ void load_rec(const PRec* __restrict__ src, double* v
 __device__ __forceinline__ void passA_body(Rows R, KickScalars* __restrict__ scp, double* __restrict__ part,
                                            const int bx, const int nbx) {
   __shared__ double lds[(kPT / 64) * 3];
-  const KickScalars s = *scp;
+  const KickScalars s = uniform_load(scp);
   double acc[3] = {0, 0, 0};
   const int64_t n = s.n;
   for (int64_t p = (int64_t)bx * kPT + threadIdx.x; p < n; p += (int64_t)nbx * kPT) {
@@ -425,7 +425,7 @@ __device__ __forceinline__ void passB_body(Rows R, const double* __restrict__ q,
   // last reader, the previous kick's z pass, ran earlier on the stream): no
   // launch and no cross-stream wait of its own
   for (int64_t i = (int64_t)bx * kPT + threadIdx.x; i < zn; i += (int64_t)nbx * kPT) zg[i] = 0ull;
-  const KickScalars s = *scp;
+  const KickScalars s = uniform_load(scp);
   const double inf = __builtin_inf();
   double mn[3] = {inf, inf, inf}, mx[3] = {-inf, -inf, -inf};
   double sq = 0, saq = 0, sqx[3] = {0, 0, 0};
@@ -710,9 +710,8 @@ __device__ __forceinline__ void deposit_body(Rows R, const double* __restrict__ 
   constexpr int kItems = DepTile<TILE>::items;
   __shared__ int hkey[kSlots];
   __shared__ long long hval[NWORD][kSlots];
-  const KickScalars& s0 = *scp;
-  if (s0.err) return;  // uniform across the grid
-  const KickScalars s = s0;
+  const KickScalars s = uniform_load(scp);
+  if (s.err) return;  // uniform across the grid
   const int64_t ncell = (int64_t)s.nmesh[0] * s.nmesh[1] * s.nmesh[2];
   unsigned long long* g = grid;
   if constexpr (XCD) g += (int64_t)xcc_id() * NWORD * ncell;
@@ -882,7 +881,7 @@ __device__ __forceinline__ void sort_keys_body(Rows R, const double* __restrict_
                                                const KickScalars* __restrict__ scp, uint32_t* __restrict__ keys,
                                                PRec* __restrict__ rec, int cells, DriftArgs ahead, uint32_t tag,
                                                const int bx, const int nbx) {
-  const KickScalars s = *scp;
+  const KickScalars s = uniform_load(scp);
   const int64_t p = (int64_t)bx * kPT + threadIdx.x;
   if (p >= s.n) return;
   double v[8];
@@ -1470,10 +1469,9 @@ __device__ __forceinline__ void kick_body(double* __restrict__ r, int64_t ld, co
                                           unsigned long long* __restrict__ zg, int64_t zn, const int bx,
                                           const int nbx) {
   __shared__ double lds[SUMP ? (kKickPT / 64) * 3 : 1];
-  const KickScalars& s0 = *scp;
-  if (s0.err) return;  // uniform across the grid
+  const KickScalars s = uniform_load(scp);
+  if (s.err) return;  // uniform across the grid
   for (int64_t i = (int64_t)bx * kKickPT + threadIdx.x; i < zn; i += (int64_t)nbx * kKickPT) zg[i] = 0ull;
-  const KickScalars s = s0;
   const int64_t blk = xcd_block(bx, nbx);
   const int64_t p = blk * kKickPT + threadIdx.x;
   const bool active = p < s.n;
