@@ -15,6 +15,14 @@
 // without a tau window pass 0's sums are pass 2's too: pass 6 = 0 + 2 + 4.
 // Every value is summed in the same order and tree as in its own pass, so the
 // results are the same bit for bit.
+//
+// A call that can wait for the host takes fewer reads (k_mom_about): sums and
+// products about a provisional centre, the mean of 64 particles spread over
+// the bunch, in one pass, and the centred moments from those:
+//   <(u - <u>)(v - <v>)> = <(u - c)(v - c')> - (<u> - c)(<v> - c')
+// which loses nothing while the centre is within about a standard deviation
+// of the mean.  Where it is not (an outlier among the 64, a window far from
+// them), the passes above run as well.
 #pragma once
 #include "particles.hpp"
 
@@ -36,6 +44,7 @@ struct MomState {
   double mom[12];     // xx, xpx, pxpx, yy, ypy, pypy, tautau, xy, pxpy, xpy, ypx, pp
   double tau_min, tau_max;  // extent of tau (slice = "Imax")
   double z0;                // window centre: mean(tau), or the peak-current position (slice = "Imax")
+  int64_t far;        // k_mom_about: the provisional centre was too far off
 };
 
 constexpr int kMomNV[8] = {2, 1, 7, 5, 4, 12, 12, 11};
@@ -217,6 +226,139 @@ __global__ void __launch_bounds__(1024) k_mom_reduce(MomState* __restrict__ msp,
       if (k < cap) table[k] = s;
       *counter = k + 1;
     }
+  }
+}
+
+// Sums about a provisional centre in one read.  DISP 0: with the dispersion
+// known, of the corrected coordinates (passes 2, 4 and 5, and pass 0's charge
+// when there is no window): count, q, the six deviations, the twelve products.
+// DISP 1: of the raw ones, for the dispersion (passes 2 and 3).
+// mb (MomAbout): the centre, written by workgroup 0 for the reduction.
+struct MomAbout {
+  double c[6];  // x, px, y, py, tau, p
+};
+constexpr int kMomAboutNV[2] = {20, 12};
+
+template <int DISP>
+__device__ __forceinline__ void mom_point(const Rows& R, int64_t i, const MomState& s, double tau, double* u) {
+  double R6[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) R6[k] = k == 4 ? tau : R.r[k * R.ld + i];
+  if constexpr (DISP == 0) {
+    mom_corrected(R6, s, &u[0], &u[2], &u[1], &u[3]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) u[k] = R6[k];
+  }
+  u[4] = tau;
+  u[5] = R6[5];
+}
+
+template <int DISP>
+__global__ void __launch_bounds__(kPT) k_mom_about(Rows R, const double* __restrict__ q,
+                                                   const MomState* __restrict__ msp, double* __restrict__ part,
+                                                   MomAbout* __restrict__ mb, MomState s0, int first) {
+  constexpr int NV = kMomAboutNV[DISP];
+  __shared__ double lds[(kPT / 64) * NV];
+  __shared__ double ctr[6];
+  const MomState s = first ? s0 : *msp;
+  // the centre: every workgroup forms the same one
+  if (threadIdx.x < 64) {
+    const int m = s.n < 64 ? (int)s.n : 64;
+    double u[6] = {0, 0, 0, 0, 0, 0};
+    if ((int)threadIdx.x < m) {
+      const int64_t i = (int64_t)threadIdx.x * (s.n / m);
+      mom_point<DISP>(R, i, s, R.r[4 * R.ld + i], u);
+    }
+    wave_reduce<6, 0>(u);
+    if (threadIdx.x == 0)
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        ctr[k] = u[k] / m;
+        if (blockIdx.x == 0) mb->c[k] = ctr[k];
+      }
+  }
+  __syncthreads();
+  const double c[6] = {ctr[0], ctr[1], ctr[2], ctr[3], ctr[4], ctr[5]};
+  double acc[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) acc[k] = 0;
+  for (int64_t i = (int64_t)blockIdx.x * kPT + threadIdx.x; i < s.n; i += (int64_t)gridDim.x * kPT) {
+    const double tau = R.r[4 * R.ld + i];
+    if (s.bounds && !(s.lo <= tau && tau <= s.hi)) continue;
+    double u[6];
+    mom_point<DISP>(R, i, s, tau, u);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) u[k] -= c[k];
+    acc[0] += 1.0;
+    if constexpr (DISP == 0) {
+      if (first) acc[1] += q[i];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) acc[2 + k] += u[k];
+      acc[8] += u[0] * u[0];
+      acc[9] += u[0] * u[1];
+      acc[10] += u[1] * u[1];
+      acc[11] += u[2] * u[2];
+      acc[12] += u[2] * u[3];
+      acc[13] += u[3] * u[3];
+      acc[14] += u[4] * u[4];
+      acc[15] += u[0] * u[2];
+      acc[16] += u[1] * u[3];
+      acc[17] += u[0] * u[3];
+      acc[18] += u[2] * u[1];
+      acc[19] += u[5] * u[5];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) acc[1 + k] += u[k];
+      acc[7] += u[5] * u[5];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[8 + k] += u[5] * u[k];
+    }
+  }
+  block_reduce<NV, 0>(acc, lds);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < NV; ++k) part[k * gridDim.x + blockIdx.x] = acc[k];
+}
+
+// totals, then the state that the passes they stand for leave; s.far: the
+// centre was further from a mean than its standard deviation
+template <int DISP>
+__global__ void __launch_bounds__(1024) k_mom_about_reduce(MomState* __restrict__ msp, const double* __restrict__ part,
+                                                           int nblk, const MomAbout* __restrict__ mb, MomState s0,
+                                                           int first) {
+  constexpr int NV = kMomAboutNV[DISP];
+  __shared__ double lds[16 * NV];
+  double t[NV];
+  reduce_partials<NV, 0>(part, nblk, t, lds);
+  if (threadIdx.x != 0) return;
+  MomState& s = *msp;
+  if (first) s = s0;
+  const double cnt = t[0];
+  s.cnt = cnt;
+  double e[6];  // mean minus centre
+  for (int k = 0; k < 6; ++k) e[k] = t[(DISP ? 1 : 2) + k] / cnt;
+  if constexpr (DISP == 0) {
+    if (first) {
+      s.sumq = t[1];
+      s.tau_all = mb->c[4] + e[4];
+      s.z0 = s.tau_all;
+    }
+    s.m[0] = mb->c[5] + e[5];
+    s.m[5] = mb->c[4] + e[4];
+    s.c[0] = mb->c[0] + e[0];
+    s.c[1] = mb->c[2] + e[2];
+    s.c[2] = mb->c[1] + e[1];
+    s.c[3] = mb->c[3] + e[3];
+    const int a[12] = {0, 0, 1, 2, 2, 3, 4, 0, 1, 0, 2, 5}, b[12] = {0, 1, 1, 2, 3, 3, 4, 2, 3, 3, 1, 5};
+    for (int k = 0; k < 12; ++k) {
+      s.mom[k] = t[8 + k] / cnt - e[a[k]] * e[b[k]];
+      if (a[k] == b[k] && !(e[a[k]] * e[a[k]] <= s.mom[k])) s.far = 1;
+    }
+  } else {
+    s.var_p = t[7] / cnt - e[5] * e[5];
+    if (!(e[5] * e[5] <= s.var_p)) s.far = 1;
+    s.m[0] = mb->c[5] + e[5];
+    for (int k = 0; k < 4; ++k) s.D[k] = (t[8 + k] / cnt - e[5] * e[k]) / s.var_p;
   }
 }
 

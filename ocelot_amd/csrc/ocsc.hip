@@ -1862,28 +1862,45 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
   }
   const int nblk = nred_blocks(c, n);
   int rc;
-  if ((rc = ensure(L.part, (size_t)12 * nblk * sizeof(double)))) return rc;
+  if ((rc = ensure(L.part, (size_t)20 * nblk * sizeof(double) + sizeof(MomAbout)))) return rc;
   MomState& h = *c->mom_host;  // read back at the end (every call waits for its copies)
   const MomState s0 = mom_start(n, (flags & OCSC_MOM_BOUNDS) ? 1 : 0,
                                 (flags & OCSC_MOM_DISP_GIVEN) ? 1 : ((flags & OCSC_MOM_AUTO_DISP) ? 2 : 0), b0, b1, disp);
   double* part = (double*)L.part.p;
+  MomAbout* const about = (MomAbout*)(part + (size_t)20 * nblk);
   const Rows R{r, ld};
   double z0 = 0;
-  if (!s0.bounds && s0.disp_mode != 2) {
-    k_mom<6><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, nullptr, 0.0, 0.0, s0);  // passes 0, 2, 4 in one read
-    k_mom_reduce<6><<<1, 1024, 0, st>>>(c->mom, part, nblk, s0);
-  } else {
+  // the window's centre and width, over all particles
+  auto window = [&]() -> int {
     k_mom<0><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, nullptr, 0.0, 0.0, s0);
     k_mom_reduce<0><<<1, 1024, 0, st>>>(c->mom, part, nblk, s0);
-    if (s0.bounds) {
-      k_mom<1><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
-      k_mom_reduce<1><<<1, 1024, 0, st>>>(c->mom, part, nblk);
-      if (flags & OCSC_MOM_IMAX) {
-        if ((rc = imax_window(c, R, n, st, &z0))) return rc;
-      } else {
-        z0 = -1;  // mean(tau), set below from the device state
-      }
+    if (!s0.bounds) return OCSC_OK;
+    k_mom<1><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
+    k_mom_reduce<1><<<1, 1024, 0, st>>>(c->mom, part, nblk);
+    return flags & OCSC_MOM_IMAX ? imax_window(c, R, n, st, &z0) : OCSC_OK;
+  };
+  auto read_back = [&]() -> int {
+    LAUNCHCHK("k_mom");
+    HIPCHK(hipMemcpyAsync(&h, c->mom, sizeof(h), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return OCSC_OK;
+  };
+  // one read of the rows (two where the dispersion is asked for) about a
+  // provisional centre
+  {
+    const int first = !s0.bounds && s0.disp_mode != 2;
+    if (!first && (rc = window())) return rc;
+    if (s0.disp_mode == 2) {
+      k_mom_about<1><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, about, s0, 0);
+      k_mom_about_reduce<1><<<1, 1024, 0, st>>>(c->mom, part, nblk, about, s0, 0);
     }
+    k_mom_about<0><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, about, s0, first);
+    k_mom_about_reduce<0><<<1, 1024, 0, st>>>(c->mom, part, nblk, about, s0, first);
+    if ((rc = read_back())) return rc;
+  }
+  if (h.far) {
+    // the centre was no centre: means first, then the moments about them
+    if ((rc = window())) return rc;
     if (s0.disp_mode != 2) {
       k_mom<7><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);  // passes 2 and 4 in one read
       k_mom_reduce<7><<<1, 1024, 0, st>>>(c->mom, part, nblk);
@@ -1895,12 +1912,10 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
       k_mom<4><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
       k_mom_reduce<4><<<1, 1024, 0, st>>>(c->mom, part, nblk);
     }
+    k_mom<5><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
+    k_mom_reduce<5><<<1, 1024, 0, st>>>(c->mom, part, nblk);
+    if ((rc = read_back())) return rc;
   }
-  k_mom<5><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);
-  k_mom_reduce<5><<<1, 1024, 0, st>>>(c->mom, part, nblk);
-  LAUNCHCHK("k_mom");
-  HIPCHK(hipMemcpyAsync(&h, c->mom, sizeof(h), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
   double v[OCSC_MOM_NOUT];
   v[0] = h.cnt;
   v[1] = h.sumq;

@@ -252,12 +252,20 @@ __device__ __forceinline__ double partials_total(const double* __restrict__ p, i
   constexpr int KIND = OP ? 1 : 0, C = OP == 2 ? 3 : 0, G = 4;
   const int lane = threadIdx.x & 63;
   const int nw = nblk < 1024 ? (nblk + 63) >> 6 : 16;
+  // the next four values (of the first 1024 partials) are loaded while these
+  // go through the lanes
+  double t[G], nxt[G];
+#pragma unroll
+  for (int k = 0; k < G; ++k) nxt[k] = lane + 64 * k < nblk ? p[lane + 64 * k] : red_id<KIND>(C);
 #pragma unroll 1
   for (int w0 = 0; w0 < nw; w0 += G) {
-    double t[G];
     const int b = lane + 64 * w0;
 #pragma unroll
-    for (int k = 0; k < G; ++k) t[k] = b + 64 * k < nblk ? p[b + 64 * k] : red_id<KIND>(C);
+    for (int k = 0; k < G; ++k) {
+      t[k] = nxt[k];
+      const int bn = b + 64 * (G + k);
+      nxt[k] = w0 + G < nw && bn < nblk ? p[bn] : red_id<KIND>(C);
+    }
 #pragma unroll 1
     for (int b1 = b + 1024; b1 < nblk; b1 += 1024)
 #pragma unroll
