@@ -331,9 +331,14 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * deposit's LDS table (fewer same-slot LDS atomics in cell order), 0
  * (default) does not; bit-identical results.  "apply_sort": one-shot kicks
  * (ocsc_apply) deposit and kick a cell-ordered copy of the bunch and write
- * the result back in the caller's order: 0 never, 1 always, 2 (default) in
- * the FP64 form from 1000000 particles on; bit-identical results
- * (ocsc_apply_cells and ocsc_apply_noalloc never sort).  "apply_resort":
+ * the result back in the caller's order: 0 never, 1 always, 2 (default) where
+ * the bricks below do not fit, in the FP64 form from 1000000 particles on.
+ * With 2, kicks of at least 450000 particles on meshes of at most 4096 bricks
+ * (16 x 16 x 16 cells, FP64 8 x 16 x 16 where that fits: up to 256 cells per
+ * axis) and default deposit options stay in the caller's order and deposit
+ * through runs of (charge, cell) per brick (24 bytes of workspace per
+ * particle).  Bit-identical results (ocsc_apply_cells and ocsc_apply_noalloc
+ * never sort and use no bricks).  "apply_resort":
  * such a kick sorts on the first of every apply_resort calls (1..1000,
  * default 10) on the same rows (pointer, particle count and row stride) and
  * the calls in between re-use that call's cell order (any order gives the

@@ -290,7 +290,7 @@ struct ocsc_ctx {
   int red_blocks = kMaxRedBlocks;  // blocks of the strided reduction passes
   int sort_every = 10;  // tracking: re-sort the resident bunch by cell every k steps (0: never)
   int permute_rec = 1;  // tracking: permutations staged through 64-byte particle records (0: row by row)
-  int apply_sort = 2;   // one-shot kicks on a cell-ordered copy: 0 never, 1 always, 2 FP64 from kApplySortMin particles
+  int apply_sort = 2;   // one-shot kicks on a cell-ordered copy: 0 never, 1 always, 2 where use_bins and kApplySortMin say
   int batch_sort = 1;   // batched calls keep a cell-ordered copy of each bunch across the kicks of a call
   int sort_cells = 1;   // sort keys: bricks and the cells inside them (1), or bricks only (0)
   int sort_ahead = 1;   // tracking sort keys at the position half-way through the re-sort interval
@@ -685,26 +685,17 @@ KickInputs kick_inputs(const int32_t* nmesh, int64_t n, double E_GeV, double zst
 // resident workgroups (no tail of half-empty rounds), at most one per 8 * 256
 // particles (every thread sums several particles before the workgroup's
 // reduction tree: the passes over a batch's bunches of a few 1e5 particles
-// take 268 us at 8 particles per thread, 305 at 2) unless that leaves CUs
-// without a workgroup: then one per CU, down to one particle per thread
-// (20k particles: pass A 9.2 -> 3.8 us, pass B 12.1 -> 5.5 us; 333k: 10.6 ->
-// 8.0 and 13.0 -> 10.7 us)
+// take 268 us at 8 particles per thread, 305 at 2).  More workgroups for small
+// bunches were faster, but another split moves the frame in its last bits: the
+// FP32 rounding of every field value with it, and in the FP64 form the smallest
+// of a tracked bunch's means by 1e-9 of themselves.
 constexpr int64_t kRedParticles = 8 * kPT;
-constexpr int64_t kRedMinBlocks = 256;  // one workgroup per CU
 int nred_blocks(const ocsc_ctx* c, int64_t n) {
-  const int64_t full = (n + kRedParticles - 1) / kRedParticles, most = (n + kPT - 1) / kPT;
-  const int64_t b = std::max(full, std::min(most, kRedMinBlocks));
-  return (int)(b < c->red_blocks ? (b < 1 ? 1 : b) : c->red_blocks);
-}
-// The frame and extent passes: the mixed form keeps 8 particles per thread at
-// every size.  Another split moves the frame in its last bits and with it the
-// FP32 rounding of every field value (1e-7 of the kick, where the FP64 form
-// moves 1e-15).
-int frame_blocks(const ocsc_ctx* c, int64_t n, int prec) {
-  if (prec == OCSC_FP64) return nred_blocks(c, n);
   const int64_t b = (n + kRedParticles - 1) / kRedParticles;
   return (int)(b < c->red_blocks ? (b < 1 ? 1 : b) : c->red_blocks);
 }
+// passes A and B with 1024 threads per workgroup while that leaves CUs free
+constexpr int64_t kSplitMax = 256 * kRedParticles;
 
 // read back one timed kick of the profiling ring
 int flush_slot(ocsc_ctx* c, int k) {
@@ -919,7 +910,7 @@ template <typename F, int NWORD>
 int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld, const double* q, const KickInputs& in,
                  int prec, hipStream_t st, const StepOpts& o = StepOpts()) {
   const int64_t n = in.n;
-  const int nblk = frame_blocks(c, n, prec);
+  const int nblk = nred_blocks(c, n);
   const int npart = (int)((n + kKickPT - 1) / kKickPT);  // kick workgroups
   Rows R{r, ld};
   const bool prof = c->profiling != 0;
@@ -972,7 +963,10 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
     double* folded = (double*)L.part.p + (size_t)3 * o.prev_nblk;
     k_fold_frame<<<kFoldBlocks, 256, 0, st>>>((const double*)L.part.p, o.prev_nblk, folded, L.sc, in);
   } else if (o.passA) {
-    k_passA<<<nblk, kPT, 0, st>>>(R, L.sc, (double*)L.part.p);
+    if (n <= kSplitMax)
+      k_passA_split<<<nblk, kSplitPT, 0, st>>>(R, L.sc, (double*)L.part.p);
+    else
+      k_passA<<<nblk, kPT, 0, st>>>(R, L.sc, (double*)L.part.p);
     k_reduceA<<<1, 1024, 0, st>>>(L.sc, (double*)L.part.p, nblk);
   } else if (o.prev_nblk > kMaxRedBlocks) {
     // one partial per kick block: fold them on many CUs first
@@ -985,10 +979,11 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   mark(1);
   // a kick that re-uses a cell order takes its particle records from pass B
   PRec* const recB = o.sort && o.sort->order_in ? o.sort->rec : nullptr;
-  if (prec == OCSC_MIXED)
-    k_passB<true><<<nblk, kPT, 0, st>>>(R, q, L.sc, (double*)L.part.p, zg, zg ? nz64 : 0, recB);
+  constexpr bool kFast = sizeof(F) == 4;
+  if (n <= kSplitMax && !recB)
+    k_passB_split<kFast><<<nblk, kSplitPT, 0, st>>>(R, q, L.sc, (double*)L.part.p, zg, zg ? nz64 : 0);
   else
-    k_passB<false><<<nblk, kPT, 0, st>>>(R, q, L.sc, (double*)L.part.p, zg, zg ? nz64 : 0, recB);
+    k_passB<kFast><<<nblk, kPT, 0, st>>>(R, q, L.sc, (double*)L.part.p, zg, zg ? nz64 : 0, recB);
   k_reduceB<<<1, 1024, 0, st>>>(L.sc, (double*)L.part.p, nblk, prec);
   LAUNCHCHK("frame/extent passes");
   mark(2);
@@ -1266,10 +1261,10 @@ int apply_via_graph(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t 
 }
 
 constexpr int kMaxLanes = 8;
-// one-shot FP64 kicks of at least this many particles go through a
-// cell-ordered copy (measured at 10M / 127^3: FP64 2.58 -> 2.42 ms, where the
-// two-word deposit's random atomics dominate; mixed 1.77 -> 2.29 ms, so the
-// mixed form stays in the caller's order)
+// Where the bricks do not fit (use_bins), one-shot FP64 kicks of at least this
+// many particles go through a cell-ordered copy (10M / 127^3 FP64 1714 us
+// directly, 1682 sorted with nine in ten calls re-using the order, 1553 through
+// bricks; mixed 1581, 1546, 1252)
 constexpr int64_t kApplySortMin = 1000000;
 
 // device address of the no-allocation workspace on `device` (current)
@@ -1637,7 +1632,7 @@ int ocsc_el_field(ocsc_ctx* c, const double* xyz, int64_t ld, const double* q, i
   } xcd_off{c, c->deposit_xcd};
   c->deposit_xcd = 0;
   in.gamma0 = gamma;
-  const int nblk = frame_blocks(c, n, prec);
+  const int nblk = nred_blocks(c, n);
   const int npart = (int)((n + kPT - 1) / kPT);
   Rows R{xyz, ld};
   k_setup<<<1, 64, 0, st>>>(L.sc, in);
@@ -2211,7 +2206,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
       // drift here; the LSC kick leaves the next kick's momentum sums, in
       // pass A's partial layout
       o.drift = o.sump = false;
-      o.prev_nblk = frame_blocks(c, n, prec);
+      o.prev_nblk = nred_blocks(c, n);
     }
     o.dr = DriftArgs{Ld, r56};
     o.ordered = sorted;
@@ -2243,7 +2238,7 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
     // the next drift: fused into the LSC kick when there are no moments
     const DriftArgs next{Ld, r56};
     const bool fuse = lq && !tw && step < nsteps - 1;
-    const LscSump sm{L.sc, (double*)L.part.p, frame_blocks(c, n, prec)};  // read by the next step's kick
+    const LscSump sm{L.sc, (double*)L.part.p, nred_blocks(c, n)};  // read by the next step's kick
     if (lq && (rc3 = enqueue_lsc(c, rr, lr, qq, n, lq->k, lq->b0, lq->b1, s2, fuse ? &next : nullptr,
                                  step < nsteps - 1 ? &sm : nullptr)))
       return rc3;
@@ -2499,7 +2494,7 @@ int fused_plan(ocsc_ctx* c, const std::vector<int>& kicked, const std::vector<do
     b.n = nn[i];
     b.sc = L.sc;
     b.part = (double*)L.part.p;
-    b.nblk = frame_blocks(c, nn[i], prec);
+    b.nblk = nred_blocks(c, nn[i]);
     b.d = g.d;
     b.ncell = g.ncell;
     b.nzero = (int64_t)ncopy * nword * g.ncell;

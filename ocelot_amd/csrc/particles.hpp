@@ -498,6 +498,102 @@ __global__ void __launch_bounds__(kPT) k_passB(Rows R, const double* __restrict_
   passB_body<FAST>(R, q, scp, part, zg, zn, blockIdx.x, gridDim.x, rec);
 }
 
+// Passes A and B of small bunches.  A thread of the strided passes adds up to
+// 8 particles one after the other, and 20k particles are 10 workgroups: the
+// passes wait for one chain of loads and transforms (9.2 and 12.1 us).  Here a
+// workgroup of 1024 threads takes the same 256 chains, four particles of each
+// at a time: every thread transforms one, and the chain's first thread adds the
+// four in the chain's order.  The same sums bit for bit.
+constexpr int kSplit = 4;
+constexpr int kSplitPT = kSplit * kPT;
+
+__global__ void __launch_bounds__(kSplitPT) k_passA_split(Rows R, const KickScalars* __restrict__ scp,
+                                                          double* __restrict__ part) {
+  __shared__ double v[kSplit][3][kPT];
+  __shared__ double lds[(kSplitPT / 64) * 3];
+  const KickScalars s = uniform_load(scp);
+  const int t = threadIdx.x % kPT, kk = threadIdx.x / kPT;
+  const int64_t n = s.n, stride = (int64_t)gridDim.x * kPT;
+  double acc[3] = {0, 0, 0};
+  for (int64_t p0 = (int64_t)blockIdx.x * kPT; p0 < n; p0 += kSplit * stride) {
+    const int64_t p = p0 + t + kk * stride;
+    if (p < n) {
+      double m[3];
+      to_p(R.r[R.ld + p], R.r[3 * R.ld + p], R.r[5 * R.ld + p], s, m);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[kk][c][t] = m[c];
+    }
+    __syncthreads();
+    if (kk == 0)
+#pragma unroll
+      for (int j = 0; j < kSplit; ++j)
+        if (p0 + t + j * stride < n)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) acc[c] += v[j][c][t];
+    __syncthreads();
+  }
+  block_reduce<3, 0>(acc, lds);
+  if (threadIdx.x == 0)
+    for (int c = 0; c < 3; ++c) part[c * gridDim.x + blockIdx.x] = acc[c];
+}
+
+template <bool FAST>
+__global__ void __launch_bounds__(kSplitPT) k_passB_split(Rows R, const double* __restrict__ q,
+                                                          KickScalars* __restrict__ scp, double* __restrict__ part,
+                                                          unsigned long long* __restrict__ zg, int64_t zn) {
+  __shared__ double v[kSplit][4][kPT];
+  __shared__ double lds[(kSplitPT / 64) * kNPartB];
+  for (int64_t i = (int64_t)blockIdx.x * kSplitPT + threadIdx.x; i < zn; i += (int64_t)gridDim.x * kSplitPT)
+    zg[i] = 0ull;
+  const KickScalars s = uniform_load(scp);
+  const int t = threadIdx.x % kPT, kk = threadIdx.x / kPT;
+  const int64_t n = s.n, stride = (int64_t)gridDim.x * kPT;
+  const double inf = __builtin_inf();
+  double a[kNPartB] = {inf, inf, inf, -inf, -inf, -inf, 0, 0, 0, 0, 0};
+  int bad = 0;
+  for (int64_t p0 = (int64_t)blockIdx.x * kPT; p0 < n; p0 += kSplit * stride) {
+    const int64_t p = p0 + t + kk * stride;
+    if (p < n) {
+      double r[6], xp[6], xyz[3];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) r[k] = ldnt(R.r + k * R.ld + p);
+      const double qq = s.q_const ? s.q_val : ldnt(q + p);
+      if constexpr (FAST)
+        to_xp_fast(r[0], r[1], r[2], r[3], r[4], r[5], s, xp);
+      else
+        to_xp(r[0], r[1], r[2], r[3], r[4], r[5], s, xp);
+      rot(xp, s.T, xyz);
+      xyz[2] = xyz[2] * s.gamma0;
+      bad |= !(__builtin_isfinite(xyz[0]) && __builtin_isfinite(xyz[1]) && __builtin_isfinite(xyz[2]) &&
+               __builtin_isfinite(qq));
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[kk][k][t] = xyz[k];
+      v[kk][3][t] = qq;
+    }
+    __syncthreads();
+    if (kk == 0)
+#pragma unroll
+      for (int j = 0; j < kSplit; ++j)
+        if (p0 + t + j * stride < n) {
+          const double qq = v[j][3][t];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            const double x = v[j][k][t];
+            a[k] = x < a[k] ? x : a[k];
+            a[3 + k] = x > a[3 + k] ? x : a[3 + k];
+            a[8 + k] += qq * x;
+          }
+          a[6] += qq;
+          a[7] += __builtin_fabs(qq);
+        }
+    __syncthreads();
+  }
+  if (bad) atomicOr(&scp->err, (int)kErrNonFinite);
+  block_reduce<kNPartB, 1>(a, lds);
+  if (threadIdx.x == 0)
+    for (int c = 0; c < kNPartB; ++c) part[c * gridDim.x + blockIdx.x] = a[c];
+}
+
 // cell sizes, grid offset, charge scale and kernel-cache decision
 // (sc.py:172-186)
 __device__ __forceinline__ void reduceB_body(KickScalars* __restrict__ scp, const double* __restrict__ part, int nblk,
