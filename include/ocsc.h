@@ -336,7 +336,7 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * With 2, kicks of at least 450000 particles on meshes of at most 4096 bricks
  * (16 x 16 x 16 cells, FP64 8 x 16 x 16 where that fits: up to 256 cells per
  * axis) and default deposit options stay in the caller's order and deposit
- * through runs of (charge, cell) per brick (24 bytes of workspace per
+ * through runs of (charge, cell) per brick (20 bytes of workspace per
  * particle).  Bit-identical results (ocsc_apply_cells and ocsc_apply_noalloc
  * never sort and use no bricks).  "apply_resort":
  * such a kick sorts on the first of every apply_resort calls (1..1000,
