@@ -348,7 +348,7 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * deposit and the kick (1, default) or gathers them into a cell-ordered
  * copy of the rows first (0); bit-identical results.  "deposit_tile": particles per thread and
  * LDS hash slots of the deposit, 0 (default) by the rows' order and number (in
- * cell order 4 and 1024, FP64 2 and 256; in the caller's order no table, one particle
+ * cell order 4 and 1024, from 1000000 particles 8 and 2048, FP64 2 and 256; in the caller's order no table, one particle
  * per thread up to 150000 and 8 above; in batches 8 and 2048, FP64 1024), 1
  * 4 and 1024 (FP64: 512), 2 16 and 4096 (FP64: 2048), 3 no table (one global atomic per particle), 4 as
  * in batches with all of a thread's particle loads issued first; bit-identical results.  "batch_sort": see
@@ -377,9 +377,10 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * bit-identical results.  The graph holds the caller's pointers: a bunch
  * freed and another allocated at the same address with the same sizes is
  * kicked correctly, since only addresses and sizes enter the sequence.
- * "grid_clear": the charge grid is cleared by the frame/extent pass B (0), on
- * the second stream where that is faster (1, default: captured one-shot kicks
- * of grids from 8 MB; else as 0), or in tracking by each step's kick for the next
+ * "grid_clear": the charge grid is cleared by the frame/extent pass B (0),
+ * where it costs least (1, default: on the second stream in captured one-shot
+ * kicks of grids from 8 MB, by the previous step's kick in mixed tracking,
+ * else as 0), or in tracking by each step's kick for the next
  * step (2; the first step of a call as 1); bit-identical results.
  * "igf_blocks": workgroups of the Green's-function node and difference
  * kernels, 0 (default) as many as their work items, 1..65536 a cap (their

@@ -295,8 +295,9 @@ struct ocsc_ctx {
   int sort_cells = 1;   // sort keys: bricks and the cells inside them (1), or bricks only (0)
   int sort_ahead = 1;   // tracking sort keys at the position half-way through the re-sort interval
   int resort_near = 0;  // re-sorts of the copy: one gather of rows, charges and permutation (1), or records
-  // charge grid cleared by pass B (0), on the second queue where that is faster
-  // (1), or in tracking by the previous step's kick (2; the first step as 1)
+  // charge grid cleared by pass B (0), where it costs least (1: pass B, the
+  // second queue, or in mixed tracking the previous step's kick), or in tracking
+  // by the previous step's kick (2; the first step as 1)
   int grid_clear = 1;
   // workgroups of the Green's-function node and difference kernels (grid-
   // stride loops; 0: one thread per node or cell): fewer leave more of the
@@ -841,12 +842,13 @@ int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // per thread up to 150k (100k: 147 either way, 200k: 162 with one, 158 with
 // eight).  In cell order the table pays (2M / 63^3 FP64 tracking step 224 us
 // with it, 351 without): the FP64 form at two particles per thread (231 with
-// eight), the mixed form at four (the first 20 steps of 10M / 127^3, whose order
-// decays fastest: 15.2 ms, 15.7 with two; later ones 14.1 with either).
-constexpr int64_t kDepOneMax = 150000;
+// eight), the mixed form at four while workgroups are few (50k / 47^3 118 us, 122
+// with eight; 2M / 63^3 208, 207) and eight above (the first 20 steps of 10M /
+// 127^3, whose order decays fastest: 15.6 ms, 15.7 with four).
+constexpr int64_t kDepOneMax = 150000, kDepWideMin = 1000000;
 int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered, int nword) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return nword == 2 ? 6 : 1;
+  if (ordered) return nword == 2 ? 6 : (n < kDepWideMin ? 1 : 0);
   return n <= kDepOneMax ? 5 : 3;
 }
 
@@ -940,8 +942,9 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // events (one-shot kicks launch by launch 23 us less in pass B at every size,
   // tracking steps 3 to 15 us).  With option grid_clear 1 a captured one-shot
   // kick of a large grid keeps the second queue, whose edges cost less in a
-  // graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  Tracking with
-  // grid_clear 2: the previous step's kick cleared it (o.grid_zeroed).
+  // graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  In mixed
+  // tracking, and with grid_clear 2, the previous step's kick cleared it
+  // (o.grid_zeroed).
   const int64_t nz64 = (c->deposit_xcd ? kNumXcd : 1) * NWORD * g.ncell;
   const bool side_clear =
       c->grid_clear && fork && capturing && o.passA && !o.sump && !o.ordered && nz64 * 8 >= kSideClearBytes;
@@ -2211,8 +2214,12 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
     o.dr = DriftArgs{Ld, r56};
     o.ordered = sorted;
     o.many = tw || lq;
-    o.grid_zeroed = c->grid_clear == 2 && step > 0;
-    o.zero_next = c->grid_clear == 2 && step < nsteps - 1;
+    // the mixed form's kick, which waits on memory, takes the clear better than
+    // its pass B (10M / 127^3 779 -> 769 us per step, smaller bunches equal), the
+    // FP64 form's pass B better than its kick (892, 900 us)
+    const bool in_kick = c->grid_clear == 2 || (c->grid_clear == 1 && prec == OCSC_MIXED);
+    o.grid_zeroed = in_kick && step > 0;
+    o.zero_next = in_kick && step < nsteps - 1;
     if (ktime) {
       o.kev0 = c->kick_ev[2 * step];
       o.kev1 = c->kick_ev[2 * step + 1];

@@ -1574,8 +1574,9 @@ __device__ __forceinline__ void kick_body(double* __restrict__ r, int64_t ld, co
                                           const int nbx) {
   __shared__ double lds[SUMP ? (kKickPT / 64) * 3 : 1];
   const KickScalars s = uniform_load(scp);
-  if (s.err) return;  // uniform across the grid
+  // (also after an error: the next step's deposit counts on a clear grid)
   for (int64_t i = (int64_t)bx * kKickPT + threadIdx.x; i < zn; i += (int64_t)nbx * kKickPT) zg[i] = 0ull;
+  if (s.err) return;  // uniform across the grid
   const int64_t blk = xcd_block(bx, nbx);
   const int64_t p = blk * kKickPT + threadIdx.x;
   const bool active = p < s.n;
