@@ -57,6 +57,14 @@ struct alignas(16) BinEntry {
   uint32_t pad;
 };
 
+// entries of chunk number `chunk` of a brick with `total` entries (one brick
+// can hold all of a bunch of up to 2^32 - 1 particles, so the rest of its
+// entries is compared unsigned)
+__host__ __device__ constexpr int bin_chunk_entries(uint32_t total, int chunk) {
+  const uint32_t left = total - (uint32_t)chunk * kBinChunk;
+  return left < (uint32_t)kBinChunk ? (int)left : kBinChunk;
+}
+
 // device buffers of one binned deposit
 struct BinBufs {
   uint32_t* keys;    // n
@@ -217,8 +225,7 @@ __global__ void __launch_bounds__(kBinPT) k_bin_deposit(const KickScalars* __res
   const int2 wk = work[blockIdx.x];
   const int words = (kBinYZ * kBinYZ * NWORD) << b.sx;
   for (int i = threadIdx.x; i < words; i += kBinPT) h[i] = 0ull;
-  const int left = (int)(T[wk.x] - (uint32_t)wk.y * kBinChunk);
-  const int cnt = left < kBinChunk ? left : kBinChunk;
+  const int cnt = bin_chunk_entries(T[wk.x], wk.y);
   const BinEntry* e0 = ent + start[wk.x] + (uint32_t)wk.y * kBinChunk;
   const double qscale = scp->qscale;
   __syncthreads();
