@@ -333,7 +333,7 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * (ocsc_apply) deposit and kick a cell-ordered copy of the bunch and write
  * the result back in the caller's order: 0 never, 1 always, 2 (default) where
  * the bricks below do not fit, in the FP64 form from 1000000 particles on.
- * With 2, kicks of at least 450000 particles on meshes of at most 4096 bricks
+ * With 2, kicks of at least 200000 particles on meshes of at most 4096 bricks
  * (16 x 16 x 16 cells, FP64 8 x 16 x 16 where that fits: up to 256 cells per
  * axis) and default deposit options stay in the caller's order and deposit
  * through runs of (charge, cell) per brick (20 bytes of workspace per
@@ -348,10 +348,10 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * deposit and the kick (1, default) or gathers them into a cell-ordered
  * copy of the rows first (0); bit-identical results.  "deposit_tile": particles per thread and
  * LDS hash slots of the deposit, 0 (default) by the rows' order and number (in
- * cell order 4 and 1024, from 1000000 particles 8 and 2048, FP64 2 and 256; in the caller's order no table, one particle
- * per thread up to 150000 and 8 above; in batches 8 and 2048, FP64 1024), 1
+ * cell order 4 and 1024, from 1000000 particles 8 and 2048, FP64 2 and 256; in the caller's order 1 and 256
+ * up to 150000, above and in batches 8 and 2048, FP64 1024), 1
  * 4 and 1024 (FP64: 512), 2 16 and 4096 (FP64: 2048), 3 no table (one global atomic per particle), 4 as
- * in batches with all of a thread's particle loads issued first; bit-identical results.  "batch_sort": see
+ * in batches, with all of a thread's particle loads issued first; bit-identical results.  "batch_sort": see
  * ocsc_apply_batched.  "fft_plan": the transform plan, 0 LDS Stockham
  * passes, radix 16 where every thread gets a butterfly (else 8), 1 radix 8
  * in every pass, 2 half as many columns per workgroup, 3 the two field

@@ -780,10 +780,11 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
 // One-shot kicks in the caller's order deposit through bricks of cells
 // (bins.hpp) from this many particles, with the default deposit options, on
 // meshes whose bricks fit a tile's histogram (up to 256 cells per axis).
-// Below, the five launches cost what the atomics do: 333k / 47x31x95 FP64 193
-// us direct, 202 through bricks; above, 500k / 63^3 209, 192; 2M / 63^3 453,
-// 354 (460, 360 launch by launch); mixed 10M / 127^3 1689, 1358.
-constexpr int64_t kApplyBinMin = 450000;
+// Below, the five launches cost what they save (through the table of dep_tile,
+// through bricks): 160k / 63^3 mixed 165, 159 us, 47x31x95 FP64 167, 160, 31^3
+// mixed 143, 146; 200k / 63^3 mixed 172, 160, 31^3 FP64 159, 153; 333k /
+// 47x31x95 FP64 203, 172; 2M / 63^3 FP64 522, 340.
+constexpr int64_t kApplyBinMin = 200000;
 bool use_bins(const ocsc_ctx* c, const Geometry& g, int nword, int64_t n) {
   return n >= kApplyBinMin && n <= (int64_t)0xFFFFFFFF && !c->deposit_tile && !c->deposit_xcd && !c->deposit_agg &&
          bin_count(bin_shape(g.d.nx, g.d.ny, g.d.nz, nword)) <= kBinMax;
@@ -835,21 +836,23 @@ int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 }
 
 // The tile the default (option deposit_tile 0, no other deposit option) takes.
-// In the caller's order a workgroup's particles share few cells, so the table
-// only delays its atomics: without it 20k / 31^3 FP64 148 -> 120 us per kick
-// (10 workgroups of 8 particles per thread left the chip idle), 200k / 63^3
-// 177 -> 158, 1.5M / 63^3 403 -> 358, 4M / 127^3 mixed 873 -> 856.  One particle
-// per thread up to 150k (100k: 147 either way, 200k: 162 with one, 158 with
-// eight).  In cell order the table pays (2M / 63^3 FP64 tracking step 224 us
-// with it, 351 without): the FP64 form at two particles per thread (231 with
-// eight), the mixed form at four while workgroups are few (50k / 47^3 118 us, 122
-// with eight; 2M / 63^3 208, 207) and eight above (the first 20 steps of 10M /
-// 127^3, whose order decays fastest: 15.6 ms, 15.7 with four).
+// Always one with a table: without it a bunch that shares few cells (a small
+// mesh, or a few far particles that stretch the mesh) waits on same-cell
+// atomics, 449k / 15^3 FP64 346 us, 145 with it; 100k / 63^3 with two particles
+// at 60 sigma 324, 160; 2M such 3914, 260.  In the caller's order one particle
+// per thread up to 150k (20k / 31^3 FP64 128 us, 155 with eight, which leave
+// the chip idle; 100k / 31^3 136, 155; 160k / 31^3 150, 158) and eight above
+// (449k / 63^3 FP64 with two particles at 60 sigma 168, 210 with one; 4M /
+// 63^3 FP64 923, 952 with four).  In cell order the FP64 form takes two
+// particles per thread (2M / 63^3 tracking step 224 us, 231 with eight), the
+// mixed form four while workgroups are few (50k / 47^3 118 us, 122 with eight;
+// 2M / 63^3 208, 207) and eight above (the first 20 steps of 10M / 127^3, whose
+// order decays fastest: 15.6 ms, 15.7 with four).
 constexpr int64_t kDepOneMax = 150000, kDepWideMin = 1000000;
 int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered, int nword) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
   if (ordered) return nword == 2 ? 6 : (n < kDepWideMin ? 1 : 0);
-  return n <= kDepOneMax ? 5 : 3;
+  return n <= kDepOneMax ? 5 : 0;
 }
 
 // the deposit variant the context's options select

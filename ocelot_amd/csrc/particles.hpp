@@ -740,17 +740,17 @@ constexpr int kDepSlots2 = 1024;             // two-word (FP64) form: half the L
 // of all of a thread's particles loaded before the first is deposited (tile
 // 0 loads one particle ahead; the deposit waits on memory most of its time)
 // Not options: tiles that the default (0) takes by itself, 5 one particle per
-// thread and no table, 6 a quarter of tile 0 (see dep_tile).
+// thread and 256 slots, 6 a quarter of tile 0 (see dep_tile).
 template <int TILE>
 struct DepTile {
-  static constexpr bool direct = TILE == 3 || TILE == 5;
+  static constexpr bool direct = TILE == 3;
   static constexpr bool all_loads = TILE == 4;  // as 0, every item's loads issued first
   static constexpr int items =
       TILE == 1 ? kDepItems / 2 : (TILE == 2 ? kDepItems * 2 : (TILE == 5 ? 1 : (TILE == 6 ? kDepItems / 4 : kDepItems)));
   template <int NWORD>
   static constexpr int slots() {
     constexpr int base = NWORD == 2 ? kDepSlots2 : kDepSlots;
-    return TILE == 1 ? base / 2 : (TILE == 2 ? base * 2 : (direct ? 1 : (TILE == 6 ? base / 4 : base)));
+    return TILE == 1 ? base / 2 : (TILE == 2 ? base * 2 : (direct ? 1 : (TILE == 5 ? kDepPT : (TILE == 6 ? base / 4 : base))));
   }
 };
 
