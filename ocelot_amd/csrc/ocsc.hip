@@ -784,9 +784,20 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
 // through bricks): 160k / 63^3 mixed 165, 159 us, 47x31x95 FP64 167, 160, 31^3
 // mixed 143, 146; 200k / 63^3 mixed 172, 160, 31^3 FP64 159, 153; 333k /
 // 47x31x95 FP64 203, 172; 2M / 63^3 FP64 522, 340.
-constexpr int64_t kApplyBinMin = 200000;
+// Not on meshes of more than 2^21 cells for few particles per cell: there the
+// many bricks cost as much as the atomics (450k / 255^3 mixed 1761 us through
+// the table, 1941 through bricks; 191^3 1245, 1261), until the mixed form has
+// one particle per two cells, where the fields go to lines (8M / 255^3 3419,
+// 3543; 8.4M 3014 before lines and bricks, 2623; 1.5M / 159^3 1170, 1131), and
+// the FP64 form, whose fields then lie beyond the 256 MB cache for the random
+// reads of a kick in the caller's order, kicks a cell-ordered copy (5M / 191^3
+// 2144 us on an order kept from an earlier call, 2314 sorting, 2361 through
+// bricks; 20M / 255^3 4916, 5637, 5784) until the sort of five particles per
+// cell costs more (35M / 191^3 6186, 7115, 6147; 50M / 159^3 8620, 10135, 7327).
+constexpr int64_t kApplyBinMin = 200000, kApplyBinCells = 1 << 21;
 bool use_bins(const ocsc_ctx* c, const Geometry& g, int nword, int64_t n) {
   return n >= kApplyBinMin && n <= (int64_t)0xFFFFFFFF && !c->deposit_tile && !c->deposit_xcd && !c->deposit_agg &&
+         (g.ncell <= kApplyBinCells || (nword == 2 ? n >= 5 * g.ncell : 2 * n >= g.ncell)) &&
          bin_count(bin_shape(g.d.nx, g.d.ny, g.d.nz, nword)) <= kBinMax;
 }
 
@@ -1267,10 +1278,9 @@ int apply_via_graph(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t 
 }
 
 constexpr int kMaxLanes = 8;
-// Where the bricks do not fit (use_bins), one-shot FP64 kicks of at least this
-// many particles go through a cell-ordered copy (10M / 127^3 FP64 1714 us
-// directly, 1682 sorted with nine in ten calls re-using the order, 1553 through
-// bricks; mixed 1581, 1546, 1252)
+// Where use_bins takes no bricks, one-shot FP64 kicks of at least this many
+// particles go through a cell-ordered copy (1M / 191^3 1648 us through the
+// table, 1578 on a kept order, 1709 sorting; 3M / 191^3 2078, 1911, 2080)
 constexpr int64_t kApplySortMin = 1000000;
 
 // device address of the no-allocation workspace on `device` (current)
