@@ -381,7 +381,8 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * "grid_clear": the charge grid is cleared by the frame/extent pass B (0),
  * where it costs least (1, default: on the second stream in captured one-shot
  * kicks of grids from 8 MB, by the previous step's kick in mixed tracking,
- * else as 0), or in tracking by each step's kick for the next
+ * by a launch of its own where fewer than 64 workgroups of the pass would
+ * clear over 512 KB each, else as 0), or in tracking by each step's kick for the next
  * step (2; the first step of a call as 1); bit-identical results.
  * "igf_blocks": workgroups of the Green's-function node and difference
  * kernels, 0 (default) as many as their work items, 1..65536 a cap (their

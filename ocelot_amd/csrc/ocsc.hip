@@ -922,6 +922,15 @@ void launch_kick(ocsc_ctx* c, Lane& L, int npart, double* r, int64_t ld, const S
 constexpr int64_t kForkCells = 65536, kForkCellsMany = 524288;
 constexpr int64_t kSideClearBytes = 8 << 20;
 
+// Whether wgs workgroups of a particle pass clear so many bytes of the charge
+// grid beside their particles in no more time than a launch of its own takes:
+// one workgroup stores 80 GB/s, 64 what the card takes.  (20k / 63^3 FP64, 400
+// KB each of 10 workgroups, 154 us either way; 50k / 95^3, 550 KB, 255 us in
+// pass B, 253 by a launch of its own; 5k / 127^3, 11 MB, 453, 312; 100k / 191^3
+// mixed, 1.1 MB each of 49, 1169, 1193; mixed tracking steps of 5k / 127^3, 820
+// KB per kick workgroup, 263, 256.)
+bool clear_rides(int64_t bytes, int64_t wgs) { return wgs >= 64 || bytes <= (int64_t)(512 << 10) * wgs; }
+
 template <typename F, int NWORD>
 int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld, const double* q, const KickInputs& in,
                  int prec, hipStream_t st, const StepOpts& o = StepOpts()) {
@@ -954,15 +963,22 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // The charge grid (all copies, all words) is cleared by pass B: its stores
   // ride on the rows' reads, where a clear on the second queue costs two more
   // events (one-shot kicks launch by launch 23 us less in pass B at every size,
-  // tracking steps 3 to 15 us).  With option grid_clear 1 a captured one-shot
-  // kick of a large grid keeps the second queue, whose edges cost less in a
-  // graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  In mixed
+  // tracking steps 3 to 15 us).  Where few workgroups meet a large grid it has
+  // a launch of its own (clear_rides).  With option grid_clear 1 a captured
+  // one-shot kick of a large grid keeps the second queue, whose edges cost less
+  // in a graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  In mixed
   // tracking, and with grid_clear 2, the previous step's kick cleared it
   // (o.grid_zeroed).
   const int64_t nz64 = (c->deposit_xcd ? kNumXcd : 1) * NWORD * g.ncell;
   const bool side_clear =
       c->grid_clear && fork && capturing && o.passA && !o.sump && !o.ordered && nz64 * 8 >= kSideClearBytes;
-  unsigned long long* const zg = side_clear || o.grid_zeroed ? nullptr : (unsigned long long*)L.grid.p;
+  const bool own_clear = c->grid_clear && !side_clear && !o.grid_zeroed && !clear_rides(nz64 * 8, nblk);
+  unsigned long long* const zg =
+      side_clear || own_clear || o.grid_zeroed ? nullptr : (unsigned long long*)L.grid.p;
+  if (own_clear) {
+    k_zero64<<<(int)std::min<int64_t>((nz64 + 255) / 256, 8192), 256, 0, st>>>((unsigned long long*)L.grid.p, nz64);
+    LAUNCHCHK("charge grid clear");
+  }
   if (side_clear) {
     HIPCHK(hipEventRecord(c->ev_fork0, st));
     HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork0, 0));
@@ -2230,7 +2246,9 @@ int track_impl(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_t n, c
     // the mixed form's kick, which waits on memory, takes the clear better than
     // its pass B (10M / 127^3 779 -> 769 us per step, smaller bunches equal), the
     // FP64 form's pass B better than its kick (892, 900 us)
-    const bool in_kick = c->grid_clear == 2 || (c->grid_clear == 1 && prec == OCSC_MIXED);
+    const int64_t grid_bytes = (int64_t)(c->deposit_xcd ? kNumXcd : 1) * (prec == OCSC_FP64 ? 2 : 1) * g.ncell * 8;
+    const bool in_kick =
+        c->grid_clear == 2 || (c->grid_clear == 1 && prec == OCSC_MIXED && clear_rides(grid_bytes, npart));
     o.grid_zeroed = in_kick && step > 0;
     o.zero_next = in_kick && step < nsteps - 1;
     if (ktime) {
