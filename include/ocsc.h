@@ -371,17 +371,16 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * the copy with one gather of rows, charges and permutation (the copy is
  * nearly in order), 0 (default) through particle records as the first sort
  * (measured faster); bit-identical results.  "apply_graph": 1 (default)
- * replays the launch sequence of ocsc_apply from a HIP graph captured at the
- * first call and kept while the particle and charge pointers, sizes, mesh,
+ * replays the launch sequence of ocsc_apply, on meshes below 65536 cells or
+ * with "overlap" = 0, from a HIP graph captured at the first call and kept while the particle and charge pointers, sizes, mesh,
  * precision, options and workspaces stay the same (energy, step and
  * random-mesh draws are updated in place), 0 launches kernel by kernel;
  * bit-identical results.  The graph holds the caller's pointers: a bunch
  * freed and another allocated at the same address with the same sizes is
  * kicked correctly, since only addresses and sizes enter the sequence.
  * "grid_clear": the charge grid is cleared by the frame/extent pass B (0),
- * where it costs least (1, default: on the second stream in captured one-shot
- * kicks of grids from 8 MB, by the previous step's kick in mixed tracking,
- * by a launch of its own where fewer than 64 workgroups of the pass would
+ * where it costs least (1, default: by the previous step's kick in mixed
+ * tracking, by a launch of its own where fewer than 64 workgroups of the pass would
  * clear over 512 KB each, else as 0), or in tracking by each step's kick for the next
  * step (2; the first step of a call as 1); bit-identical results.
  * "igf_blocks": workgroups of the Green's-function node and difference

@@ -273,7 +273,6 @@ struct ocsc_ctx {
   hipStream_t cap_stream = nullptr;  // stream used for graph capture
   hipStream_t side = nullptr;        // second stream: kernel spectrum next to the deposit
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  hipEvent_t ev_fork0 = nullptr, ev_zero = nullptr;  // charge-grid clear on the side stream (grid_clear 1)
   int overlap = 1;                   // 1: build the kernel spectrum concurrently with the deposit
   // stage timing (ocsc_set_profiling): events between the stages of a kick
   int profiling = 0;
@@ -295,8 +294,8 @@ struct ocsc_ctx {
   int sort_cells = 1;   // sort keys: bricks and the cells inside them (1), or bricks only (0)
   int sort_ahead = 1;   // tracking sort keys at the position half-way through the re-sort interval
   int resort_near = 0;  // re-sorts of the copy: one gather of rows, charges and permutation (1), or records
-  // charge grid cleared by pass B (0), where it costs least (1: pass B, the
-  // second queue, or in mixed tracking the previous step's kick), or in tracking
+  // charge grid cleared by pass B (0), where it costs least (1: pass B, a launch
+  // of its own, or in mixed tracking the previous step's kick), or in tracking
   // by the previous step's kick (2; the first step as 1)
   int grid_clear = 1;
   // workgroups of the Green's-function node and difference kernels (grid-
@@ -918,9 +917,8 @@ void launch_kick(ocsc_ctx* c, Lane& L, int npart, double* r, int64_t ld, const S
 }
 
 // cells from which the kernel spectrum is built on the second queue, and in a
-// loop with many other launches; bytes from which a captured clear is there
+// loop with many other launches
 constexpr int64_t kForkCells = 65536, kForkCellsMany = 524288;
-constexpr int64_t kSideClearBytes = 8 << 20;
 
 // Whether wgs workgroups of a particle pass clear so many bytes of the charge
 // grid beside their particles in no more time than a launch of its own takes:
@@ -953,8 +951,7 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // deposit and the z and y passes run; the main stream waits for it only
   // before the x pass, its first reader.
   // Not for small meshes, whose spectrum takes less time than the second
-  // queue's events: 20k / 31^3 FP64 kick 137 -> 115 us in line (115 -> 113 from
-  // a graph), 200k / 31^3 153 -> 144; 800k / 63^3 214 us beside the deposit, 226
+  // queue's events: 20k / 31^3 FP64 kick 137 -> 115 us in line, 200k / 31^3 153 -> 144; 800k / 63^3 214 us beside the deposit, 226
   // in line.  Launch by launch in a loop of many other launches (LSC, moments)
   // the events are host time too: 800k / 63x63x95 377 us per step beside, 364 in
   // line.
@@ -964,27 +961,14 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // ride on the rows' reads, where a clear on the second queue costs two more
   // events (one-shot kicks launch by launch 23 us less in pass B at every size,
   // tracking steps 3 to 15 us).  Where few workgroups meet a large grid it has
-  // a launch of its own (clear_rides).  With option grid_clear 1 a captured
-  // one-shot kick of a large grid keeps the second queue, whose edges cost less
-  // in a graph (800k / 127^3 FP64, 33 MB: 414 us, 430 in pass B).  In mixed
-  // tracking, and with grid_clear 2, the previous step's kick cleared it
-  // (o.grid_zeroed).
+  // a launch of its own (clear_rides).  In mixed tracking, and with grid_clear
+  // 2, the previous step's kick cleared it (o.grid_zeroed).
   const int64_t nz64 = (c->deposit_xcd ? kNumXcd : 1) * NWORD * g.ncell;
-  const bool side_clear =
-      c->grid_clear && fork && capturing && o.passA && !o.sump && !o.ordered && nz64 * 8 >= kSideClearBytes;
-  const bool own_clear = c->grid_clear && !side_clear && !o.grid_zeroed && !clear_rides(nz64 * 8, nblk);
-  unsigned long long* const zg =
-      side_clear || own_clear || o.grid_zeroed ? nullptr : (unsigned long long*)L.grid.p;
+  const bool own_clear = c->grid_clear && !o.grid_zeroed && !clear_rides(nz64 * 8, nblk);
+  unsigned long long* const zg = own_clear || o.grid_zeroed ? nullptr : (unsigned long long*)L.grid.p;
   if (own_clear) {
     k_zero64<<<(int)std::min<int64_t>((nz64 + 255) / 256, 8192), 256, 0, st>>>((unsigned long long*)L.grid.p, nz64);
     LAUNCHCHK("charge grid clear");
-  }
-  if (side_clear) {
-    HIPCHK(hipEventRecord(c->ev_fork0, st));
-    HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork0, 0));
-    k_zero64<<<(int)std::min<int64_t>((nz64 + 255) / 256, 8192), 256, 0, c->side>>>(
-        (unsigned long long*)L.grid.p, nz64);
-    HIPCHK(hipEventRecord(c->ev_zero, c->side));
   }
   mark(0);
   const bool fold_frame = !o.passA && o.prev_nblk > kMaxRedBlocks && c->fold_frame;
@@ -1026,7 +1010,6 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
     HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
     if ((rc = launch_kernel_spectrum<F>(c, L, g, c->side, 0))) return rc;
     HIPCHK(hipEventRecord(c->ev_join, c->side));
-    if (side_clear) HIPCHK(hipStreamWaitEvent(st, c->ev_zero, 0));
   }
   // one-shot kick on a cell-ordered copy: the frame and extent above came
   // from the caller's order, the deposit sums integers and the kick is per
@@ -1215,9 +1198,10 @@ void drop_apply_graph(ocsc_ctx* c) {
   for (auto& A : c->ag) drop_apply_slot(A);
 }
 
-// One-shot kick from a captured graph.  A kick is some 30 launches, many of
+// One-shot kick from a captured graph.  A kick is some 20 launches, many of
 // them a few microseconds long; launched one by one after the host has waited
-// for the previous kick, the GPU idles between them.  The sequence depends on
+// for the previous kick, the GPU idles between them where the host is slow.
+// The sequence depends on
 // the caller's pointers and sizes, the mesh, the precision, the options and
 // the workspace addresses; while those are unchanged the graph is replayed,
 // with only the set-up node's inputs (energy, step, random-mesh draws)
@@ -1383,9 +1367,7 @@ int ocsc_create(ocsc_ctx** out, int device) {
     return cleanup(fail(OCSC_EHIP, "stream"));
   if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess) return cleanup(fail(OCSC_EHIP, "stream"));
   if (hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_fork0, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_zero, hipEventDisableTiming) != hipSuccess)
+      hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess)
     return cleanup(fail(OCSC_EHIP, "event"));
   *out = c;
   return OCSC_OK;
@@ -1421,8 +1403,6 @@ int ocsc_destroy(ocsc_ctx* c) {
   if (c->side) (void)hipStreamDestroy(c->side);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-  if (c->ev_fork0) (void)hipEventDestroy(c->ev_fork0);
-  if (c->ev_zero) (void)hipEventDestroy(c->ev_zero);
   for (auto& set : c->ev)
     for (hipEvent_t e : set)
       if (e) (void)hipEventDestroy(e);
@@ -1505,7 +1485,13 @@ int ocsc_apply_cells(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_
   }
   o.lines = !o.sort && line_fields(L, g, n, prec);
   if (!L.phi.p || (prec == OCSC_FP64 && !L.E64.p)) return fail(OCSC_ENOMEM, "field workspace");
-  if (c->apply_graph && !cells && !c->profiling)
+  // From a graph while the kick is on one queue.  The two branches that larger
+  // meshes have overlap less when a graph replays them: 2M / 63^3 FP64 364 us from
+  // a graph, 334 launched one by one (2M / 47^3 351, 322; 2M / 95^3 518, 465; 2M /
+  // 127^3 617, 575; 10M / 127^3 mixed 1231, 1191; on one queue 2M / 31^3 306, 300,
+  // 20k / 31^3 126, 125).
+  const bool one_queue = !(c->overlap && g.ncell >= kForkCells);
+  if (c->apply_graph && one_queue && !cells && !c->profiling)
     rc = apply_via_graph(c, L, g, r, ld, q, in, prec, st, o);
   else
     rc = enqueue_kick_prec(c, L, g, r, ld, q, in, prec, st, o);
