@@ -21,6 +21,7 @@
 #include "sort.hpp"
 #include "batch.hpp"
 #include "bins.hpp"
+#include "buf.hpp"
 
 using namespace ocsc;
 
@@ -45,11 +46,6 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess) return fail(OCSC_EHIP, std::string(what) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-struct Buf {
-  void* p = nullptr;
-  size_t cap = 0;
-};
-
 // counts device (re)allocations of workspaces: a captured launch sequence
 // holds the addresses it was captured with and is valid while this is unchanged
 std::atomic<uint64_t> g_alloc_gen{0};
@@ -70,6 +66,26 @@ int ensure(Buf& b, size_t bytes) {
   b.cap = bytes;
   return OCSC_OK;
 }
+
+// device memory, for grow_optional
+struct DeviceMem {
+  size_t available() {
+    size_t have = 0, all = 0;
+    return hipMemGetInfo(&have, &all) == hipSuccess ? have : 0;
+  }
+  bool take(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    g_alloc_gen.fetch_add(1);
+    return true;
+  }
+  void give(void* p) {
+    (void)hipDeviceSynchronize();
+    (void)hipFree(p);
+  }
+};
 
 int next_pow2(int v) {
   int m = 1;
@@ -809,15 +825,12 @@ bool line_fields(Lane& L, const Geometry& g, int64_t n, int prec) {
   const MeshDims& d = g.d;
   if (2 * n < g.ncell || (prec == OCSC_FP64 && g.ncell * 24 < (16 << 20))) return false;
   Buf& b = prec == OCSC_FP64 ? L.E64 : L.phi;
-  const size_t grids = b.cap, lines = prec == OCSC_FP64 ? FieldLine<double>::bytes(d.nx, d.ny, d.nz)
-                                                        : FieldLine<float>::bytes(d.nx, d.ny, d.nz);
-  if (ensure(b, lines) == OCSC_OK) return true;
-  (void)ensure(b, grids);  // what it had
-  return false;
+  return grow_optional(b, prec == OCSC_FP64 ? FieldLine<double>::bytes(d.nx, d.ny, d.nz)
+                                            : FieldLine<float>::bytes(d.nx, d.ny, d.nz), DeviceMem());
 }
 
-// workspaces of the binned deposit, one allocation
-int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
+// workspaces of the binned deposit, one allocation; false where it is refused
+bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
   const int64_t nb = bin_count(bin_shape(g.d.nx, g.d.ny, g.d.nz, nword));
   // tiles: whole rounds of four workgroups per CU, at least 4 particles per
   // thread and at most 24, more where a tile would hold few of each brick
@@ -833,8 +846,7 @@ int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
     at[k] = off;
     off += (parts[k] + 255) & ~(size_t)255;
   }
-  int rc;
-  if ((rc = ensure(L.bins, off))) return rc;
+  if (!grow_optional(L.bins, off, DeviceMem())) return false;
   char* p = (char*)L.bins.p;
   B->ent = (BinEntry*)(p + at[0]);
   B->keys = (uint32_t*)(p + at[1]);
@@ -842,7 +854,7 @@ int bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
   B->start = (uint32_t*)(p + at[3]);
   B->nwork = (int*)(p + at[4]);
   B->work = (int2*)(p + at[5]);
-  return OCSC_OK;
+  return true;
 }
 
 // The tile the default (option deposit_tile 0, no other deposit option) takes.
@@ -1459,7 +1471,7 @@ int ocsc_apply_cells(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_
   BinBufs bb{};
   const int nword = prec == OCSC_FP64 ? 2 : 1;
   const bool binned = c->apply_sort == 2 && !cells && use_bins(c, g, nword, n);
-  if (binned && bin_buffers(L, g, nword, n, &bb) == OCSC_OK) {
+  if (binned && bin_buffers(L, g, nword, n, &bb)) {
     o.bins = &bb;
   } else if (!cells && n <= (int64_t)0xFFFFFFFF &&
       (c->apply_sort == 1 || (c->apply_sort == 2 && prec == OCSC_FP64 && n >= kApplySortMin))) {
@@ -1484,7 +1496,6 @@ int ocsc_apply_cells(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_
     o.sort = &sb;
   }
   o.lines = !o.sort && line_fields(L, g, n, prec);
-  if (!L.phi.p || (prec == OCSC_FP64 && !L.E64.p)) return fail(OCSC_ENOMEM, "field workspace");
   // From a graph while the kick is on one queue.  The two branches that larger
   // meshes have overlap less when a graph replays them: 2M / 63^3 FP64 364 us from
   // a graph, 334 launched one by one (2M / 47^3 351, 322; 2M / 95^3 518, 465; 2M /
