@@ -332,9 +332,9 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * (default) does not; bit-identical results.  "apply_sort": one-shot kicks
  * (ocsc_apply) deposit and kick a cell-ordered copy of the bunch and write
  * the result back in the caller's order: 0 never, 1 always, 2 (default) in the
- * FP64 form from 1000000 particles on where no bricks are taken.  With 2 and
- * default deposit options, kicks of at least 200000 particles stay in the
- * caller's order and deposit through runs of (charge, cell) per brick of 16 x
+ * FP64 form from 1000000 particles on where no bricks are taken.  With 2,
+ * kicks of at least 200000 particles stay in the
+ * caller's order and deposit, whatever the deposit options, through runs of (charge, cell) per brick of 16 x
  * 16 x 16 cells (FP64 8 x 16 x 16 where that fits; 20 bytes of workspace per
  * particle) on meshes of at most 4096 bricks and 2^21 cells; on meshes of more
  * cells from one particle per two cells (FP64 five per cell) on.

@@ -15,8 +15,9 @@ Knobs (``ocsc_set_option``):
 * ``deposit_agg``: runs of equal cells summed across the wavefront before
   the deposit's LDS table;
 * ``deposit_tile``: particles per thread and LDS hash slots of the deposit
-  (0: 8 x 2048, 1: 4 x 1024, 2: 16 x 4096, 4: as 0 with every particle's
-  loads issued first);
+  (0: 2 x 256 in the FP64 form, 8 x 2048 from a million particles in the mixed
+  form, below as 1; 1: 4 x 1024 (FP64 512), 2: 16 x 4096 (FP64 2048), 4: 8 x
+  2048 (FP64 1024) with every particle's loads issued first);
 * ``permute_rec``: permutations of the tracking copy through 64-byte
   particle records or row by row;
 * ``overlap``: Green's-function spectrum on a second stream next to the
@@ -38,7 +39,8 @@ precision, device) and in a JSON file keyed by GPU architecture, mesh,
 precision and bunch-size bucket (a power of two), so another process on the
 same kind of GPU re-applies them without measuring: ``$OCSC_AUTOTUNE_CACHE``
 or ``~/.cache/ocelot_amd/autotune.json`` (``OCSC_AUTOTUNE_CACHE=""`` turns
-the file off).
+the file off).  The deposit options tuned here do not reach the one-shot kicks that
+deposit through bricks of cells.
 
 ``SpaceCharge(autotune=True)`` runs this at the start of ``track_drift``.
 """
@@ -56,6 +58,10 @@ DEFAULT_SPACE = {"sort_every": (5, 7, 10, 14, 20), "sort_ahead": (0, 1), "deposi
                  "deposit_agg": (0, 1), "deposit_tile": (0, 1, 2, 4), "permute_rec": (0, 1), "overlap": (0, 1),
                  "fft_plan": (0, 1, 2, 3, 4)}
 BIT_IDENTICAL = ("deposit_xcd", "deposit_agg", "deposit_tile", "permute_rec", "overlap")
+
+# entries of the file with another version were measured when an option value
+# stood for other kernels (2: deposit_tile 0 as above) and are measured again
+FILE_VERSION = 2
 
 _cache = {}
 _file_lock = threading.Lock()
@@ -163,7 +169,7 @@ def tune_tracking(p_array, sc, L, dz, steps=30, space=None, check_bits=True, for
         if key in _cache:
             return apply(_cache[key], "memory")
         entry = load_file().get(fkey) if use_file else None
-        if entry and set(entry.get("options", {})) >= set(space):
+        if entry and entry.get("version") == FILE_VERSION and set(entry.get("options", {})) >= set(space):
             entry = {**entry, "options": {k: entry["options"][k] for k in space}}
             _cache[key] = entry
             return apply(entry, "file")
@@ -195,7 +201,7 @@ def tune_tracking(p_array, sc, L, dz, steps=30, space=None, check_bits=True, for
     out = {"options": best,
            "ms_per_step": round(min(t for tm in timings.values() for t in tm.values()) * 1e3, 4),
            "timings_ms": {k: {str(v): round(t * 1e3, 4) for v, t in tm.items()} for k, tm in timings.items()},
-           "steps": steps, "particles": n}
+           "steps": steps, "particles": n, "version": FILE_VERSION}
     _cache[key] = out
     if use_file:
         store_file(fkey, out)

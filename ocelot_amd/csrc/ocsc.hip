@@ -793,8 +793,10 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
 }
 
 // One-shot kicks in the caller's order deposit through bricks of cells
-// (bins.hpp) from this many particles, with the default deposit options, on
-// meshes whose bricks fit a tile's histogram (up to 256 cells per axis).
+// (bins.hpp) from this many particles on meshes whose bricks fit a tile's
+// histogram.  The deposit options, which the tracking autotuner sets for its
+// cell-ordered copy, have no say: with deposit_tile 4 instead of 0 a 2M / 63^3
+// FP64 kick on the context took 495 us, 334 through bricks.
 // Below, the five launches cost what they save (through the table of dep_tile,
 // through bricks): 160k / 63^3 mixed 165, 159 us, 47x31x95 FP64 167, 160, 31^3
 // mixed 143, 146; 200k / 63^3 mixed 172, 160, 31^3 FP64 159, 153; 333k /
@@ -810,8 +812,8 @@ void launch_deposit_t(Rows R, const double* q, KickScalars* sc, unsigned long lo
 // bricks; 20M / 255^3 4916, 5637, 5784) until the sort of five particles per
 // cell costs more (35M / 191^3 6186, 7115, 6147; 50M / 159^3 8620, 10135, 7327).
 constexpr int64_t kApplyBinMin = 200000, kApplyBinCells = 1 << 21;
-bool use_bins(const ocsc_ctx* c, const Geometry& g, int nword, int64_t n) {
-  return n >= kApplyBinMin && n <= (int64_t)0xFFFFFFFF && !c->deposit_tile && !c->deposit_xcd && !c->deposit_agg &&
+bool use_bins(const Geometry& g, int nword, int64_t n) {
+  return n >= kApplyBinMin && n <= (int64_t)0xFFFFFFFF &&
          (g.ncell <= kApplyBinCells || (nword == 2 ? n >= 5 * g.ncell : 2 * n >= g.ncell)) &&
          bin_count(bin_shape(g.d.nx, g.d.ny, g.d.nz, nword)) <= kBinMax;
 }
@@ -1470,7 +1472,7 @@ int ocsc_apply_cells(ocsc_ctx* c, double* r, int64_t ld, const double* q, int64_
   bool reuse = false, keep = false;
   BinBufs bb{};
   const int nword = prec == OCSC_FP64 ? 2 : 1;
-  const bool binned = c->apply_sort == 2 && !cells && use_bins(c, g, nword, n);
+  const bool binned = c->apply_sort == 2 && !cells && use_bins(g, nword, n);
   if (binned && bin_buffers(L, g, nword, n, &bb)) {
     o.bins = &bb;
   } else if (!cells && n <= (int64_t)0xFFFFFFFF &&
