@@ -3169,6 +3169,7 @@ int ocsc_apply_batched(ocsc_ctx* c, const ocsc_bunch* b, int nb, int prec, int n
         rr = sbs[i].rs;
         ldr = b[i].n;
         qq = sbs[i].qs;
+        o.ordered = true;
       }
       if ((r2 = enqueue_kick_prec(c, L, geo[i], rr, ldr, qq, ins[i], prec, L.stream, o))) return r2;
     }
