@@ -87,6 +87,24 @@ struct DeviceMem {
   }
 };
 
+// A graph of this call and its executable: given up when the call returns, after
+// the launches that are still running.
+struct CallGraph {
+  hipStream_t st;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  explicit CallGraph(hipStream_t s) : st(s) {}
+  CallGraph(const CallGraph&) = delete;
+  CallGraph& operator=(const CallGraph&) = delete;
+  ~CallGraph() {
+    if (exec) {
+      (void)hipStreamSynchronize(st);
+      (void)hipGraphExecDestroy(exec);
+    }
+    if (graph) (void)hipGraphDestroy(graph);
+  }
+};
+
 int next_pow2(int v) {
   int m = 1;
   while (m < v) m <<= 1;
@@ -2925,23 +2943,17 @@ int apply_batched_fused(ocsc_ctx* c, const ocsc_bunch* b, int nb, const std::vec
     if ((rc = fused_back_prec(c, ps, prec, st))) return rc;
     first = 1;
   }
+  CallGraph rounds(st);
   if (!use_graph || nkicks - first < 2) {
     for (int k = first; k < nkicks; ++k)
       if ((rc = fused_round_prec(c, later, prec, st))) return rc;
   } else {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
     HIPCHK(hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal));
     const int r2 = fused_round_prec(c, later, prec, c->cap_stream);
-    hipError_t e = hipStreamEndCapture(c->cap_stream, &graph);
-    if (r2 || e != hipSuccess) {
-      if (graph) (void)hipGraphDestroy(graph);
-      return r2 ? r2 : fail(OCSC_EHIP, std::string("batched capture: ") + hipGetErrorString(e));
-    }
-    e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    for (int k = first; k < nkicks && e == hipSuccess; ++k) e = hipGraphLaunch(exec, st);
-    if (exec) (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    hipError_t e = hipStreamEndCapture(c->cap_stream, &rounds.graph);
+    if (r2 || e != hipSuccess) return r2 ? r2 : fail(OCSC_EHIP, std::string("batched capture: ") + hipGetErrorString(e));
+    e = hipGraphInstantiate(&rounds.exec, rounds.graph, nullptr, nullptr, 0);
+    for (int k = first; k < nkicks && e == hipSuccess; ++k) e = hipGraphLaunch(rounds.exec, st);
     if (e != hipSuccess) return fail(OCSC_EHIP, std::string("batched graph: ") + hipGetErrorString(e));
   }
   if (copy) {
@@ -3202,6 +3214,7 @@ int ocsc_apply_batched(ocsc_ctx* c, const ocsc_bunch* b, int nb, int prec, int n
     }
   }
   const int first_graph_round = (!use_graph || any_sorted) ? 1 : 0;
+  CallGraph rounds(st);
   if (!use_graph) {
     for (int k = 1; k < nkicks; ++k)
       if ((rc = round(st, false))) {
@@ -3209,24 +3222,19 @@ int ocsc_apply_batched(ocsc_ctx* c, const ocsc_bunch* b, int nb, int prec, int n
         return rc;
       }
   } else if (nkicks > first_graph_round) {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
     hipError_t e = hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
       restore();
       return fail(OCSC_EHIP, std::string("capture: ") + hipGetErrorString(e));
     }
     int r2 = round(c->cap_stream, !any_sorted);
-    e = hipStreamEndCapture(c->cap_stream, &graph);
+    e = hipStreamEndCapture(c->cap_stream, &rounds.graph);
     if (r2 || e != hipSuccess) {
-      if (graph) (void)hipGraphDestroy(graph);
       restore();
       return r2 ? r2 : fail(OCSC_EHIP, std::string("capture: ") + hipGetErrorString(e));
     }
-    e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    for (int k = first_graph_round; k < nkicks && e == hipSuccess; ++k) e = hipGraphLaunch(exec, st);
-    if (exec) (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    e = hipGraphInstantiate(&rounds.exec, rounds.graph, nullptr, nullptr, 0);
+    for (int k = first_graph_round; k < nkicks && e == hipSuccess; ++k) e = hipGraphLaunch(rounds.exec, st);
     if (e != hipSuccess) {
       restore();
       return fail(OCSC_EHIP, std::string("batched graph: ") + hipGetErrorString(e));
