@@ -1906,12 +1906,12 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
   }
   const int nblk = nred_blocks(c, n);
   int rc;
-  if ((rc = ensure(L.part, (size_t)20 * nblk * sizeof(double) + sizeof(MomAbout)))) return rc;
+  if ((rc = ensure(L.part, (size_t)kMomAboutNV[0] * nblk * sizeof(double) + sizeof(MomAbout)))) return rc;
   MomState& h = *c->mom_host;  // read back at the end (every call waits for its copies)
   const MomState s0 = mom_start(n, (flags & OCSC_MOM_BOUNDS) ? 1 : 0,
                                 (flags & OCSC_MOM_DISP_GIVEN) ? 1 : ((flags & OCSC_MOM_AUTO_DISP) ? 2 : 0), b0, b1, disp);
   double* part = (double*)L.part.p;
-  MomAbout* const about = (MomAbout*)(part + (size_t)20 * nblk);
+  MomAbout* const about = (MomAbout*)(part + (size_t)kMomAboutNV[0] * nblk);
   const Rows R{r, ld};
   double z0 = 0;
   // the window's centre and width, over all particles
@@ -1930,10 +1930,13 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
     return OCSC_OK;
   };
   // one read of the rows (two where the dispersion is asked for) about a
-  // provisional centre
-  {
-    const int first = !s0.bounds && s0.disp_mode != 2;
-    if (!first && (rc = window())) return rc;
+  // provisional centre; not for windows that would hold less than a twelfth of
+  // a Gaussian bunch, whose passes are short and whose particles the sample
+  // for the centre mostly misses
+  const int first = !s0.bounds && s0.disp_mode != 2;
+  const bool narrow = s0.bounds && 0.5 * (std::erf(b1 * M_SQRT1_2) - std::erf(b0 * M_SQRT1_2)) < 0.08;
+  if (!first && (rc = window())) return rc;
+  if (!narrow) {
     if (s0.disp_mode == 2) {
       k_mom_about<1><<<nblk, kPT, 0, st>>>(R, q, c->mom, part, about, s0, 0);
       k_mom_about_reduce<1><<<1, 1024, 0, st>>>(c->mom, part, nblk, about, s0, 0);
@@ -1942,9 +1945,10 @@ int ocsc_moments(ocsc_ctx* c, const double* r, int64_t ld, const double* q, int6
     k_mom_about_reduce<0><<<1, 1024, 0, st>>>(c->mom, part, nblk, about, s0, first);
     if ((rc = read_back())) return rc;
   }
-  if (h.far) {
-    // the centre was no centre: means first, then the moments about them
-    if ((rc = window())) return rc;
+  if (narrow || h.far) {
+    // no centre, or it was none: means first, then the moments about them (the
+    // window, if it has been formed, stands)
+    if (first && (rc = window())) return rc;
     if (s0.disp_mode != 2) {
       k_mom<7><<<nblk, kPT, 0, st>>>(R, q, c->mom, part);  // passes 2 and 4 in one read
       k_mom_reduce<7><<<1, 1024, 0, st>>>(c->mom, part, nblk);
