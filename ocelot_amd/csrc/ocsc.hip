@@ -853,7 +853,10 @@ bool line_fields(Lane& L, const Geometry& g, int64_t n, int prec) {
 bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
   const int64_t nb = bin_count(bin_shape(g.d.nx, g.d.ny, g.d.nz, nword));
   // tiles: whole rounds of four workgroups per CU, at least 4 particles per
-  // thread and at most 24, more where a tile would hold few of each brick
+  // thread and at most 24, from 768 bricks on one per 32 bricks, since a tile
+  // writes a run per brick (50M / 255^3 mixed, 4096 bricks: 8747 us at 24, 8536
+  // at 48, 8394 at 128; 50M / 191^3 FP64, 3456: 8219, 8091, 8077; from 31^3 to
+  // 127^3 within a per cent from 12 to 128)
   const int64_t most = std::max<int64_t>(24, nb / 32);
   const int64_t round = (int64_t)kBinTilePT * 1024, rounds = (n + most * round - 1) / (most * round);
   B->items = (int)std::max<int64_t>(4, (n + rounds * round - 1) / (rounds * round));
@@ -885,15 +888,16 @@ bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // per thread up to 150k (20k / 31^3 FP64 128 us, 155 with eight, which leave
 // the chip idle; 100k / 31^3 136, 155; 160k / 31^3 150, 158) and eight above
 // (449k / 63^3 FP64 with two particles at 60 sigma 168, 210 with one; 4M /
-// 63^3 FP64 923, 952 with four).  In cell order the FP64 form takes two
-// particles per thread (2M / 63^3 tracking step 224 us, 231 with eight), the
-// mixed form four while workgroups are few (50k / 47^3 118 us, 122 with eight;
-// 2M / 63^3 208, 207) and eight above (the first 20 steps of 10M / 127^3, whose
-// order decays fastest: 15.6 ms, 15.7 with four).
-constexpr int64_t kDepOneMax = 150000, kDepWideMin = 1000000;
-int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered, int nword) {
+// 63^3 FP64 923, 952 with four).  In cell order two particles per thread in both
+// forms (us per step of a first call of 20, with two, four, eight: 50k / 31^3
+// mixed 95, 98, 101, FP64 97, 104, 108; 2M / 63^3 mixed 203, 207, 204, FP64 220,
+// 227, 225; 5M / 127^3 mixed 492, 494, 497; 10M / 127^3 mixed 722, 721, 728; the
+// most it loses is 1.5 per cent against eight, at 1M to 2M / 127^3 mixed, 354, 361,
+// 351).
+constexpr int64_t kDepOneMax = 150000;
+int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return nword == 2 ? 6 : (n < kDepWideMin ? 1 : 0);
+  if (ordered) return 6;
   return n <= kDepOneMax ? 5 : 0;
 }
 
@@ -902,7 +906,7 @@ template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
                     int32_t* cells, int64_t n, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = dep_tile(c, n, ordered, NWORD);
+  const int t = dep_tile(c, n, ordered);
   if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
   if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \
@@ -985,8 +989,11 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   // Not for small meshes, whose spectrum takes less time than the second
   // queue's events: 20k / 31^3 FP64 kick 137 -> 115 us in line, 200k / 31^3 153 -> 144; 800k / 63^3 214 us beside the deposit, 226
   // in line.  Launch by launch in a loop of many other launches (LSC, moments)
-  // the events are host time too: 800k / 63x63x95 377 us per step beside, 364 in
-  // line.
+  // the events are host time too, and the line lies higher (us per step beside,
+  // in line): with LSC and moments 800k / 63x63x95 330, 316, 800k / 95^3 421, 418,
+  // 800k / 127^3 504, 505, 2M / 79^3 503, 501, 2M / 127^3 613, 617; with moments
+  // alone, fewer launches, 800k / 63x63x95 238, 237, 2M / 79^3 386, 398, 50k / 127^3
+  // 348, 349.
   const bool capturing = st == c->cap_stream;
   const bool fork = c->overlap && !prof && g.ncell >= (o.many && !capturing ? kForkCellsMany : kForkCells);
   // The charge grid (all copies, all words) is cleared by pass B: its stores

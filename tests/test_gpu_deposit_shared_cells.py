@@ -53,6 +53,21 @@ def test_shared_cells_give_the_bits_of_the_plain_atomics(n, mesh, far, prec):
     assert all(torch.equal(out[0], o) for o in out[1:])
 
 
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [511, 513, 1_000_001])
+def test_cell_order_with_the_kicks_clear(n, prec):
+    """Tracking steps after the first deposit into the grid that the mixed form's
+    kick has cleared: the same bits with every tile, and with pass B's clear."""
+    from ocelot_amd import SpaceCharge, track_drift
+    out = []
+    for opts in (dict(), dict(deposit_tile=2), dict(deposit_tile=3), dict(grid_clear=0)):
+        d = _bunch(n, 0)
+        with _options(**opts):
+            track_drift(d, SpaceCharge(nmesh_xyz=[17, 19, 15], precision=prec), L=0.1, dz=0.1, nsteps=4)
+        out.append(d.rparticles.clone())
+    assert all(torch.equal(out[0], o) for o in out[1:])
+
+
 def _kick_ms(n, far, prec, reps=15):
     from ocelot_amd import SpaceCharge
     d, sc = _bunch(n, far), SpaceCharge(nmesh_xyz=[63] * 3, precision=prec)
