@@ -146,7 +146,7 @@ def _kick(proc, p_array, zstep, want_cells):
         host = torch.from_numpy(r if direct else np.ascontiguousarray(r, dtype=np.float64))
         ctx = _lib.context(dev)
         both = ctx.upload((host, torch.from_numpy(np.ascontiguousarray(p_array.q_array, dtype=np.float64))))
-        rt, qt = both[:6 * n], both[6 * n:]
+        rt, qt = both[:host.numel()], both[host.numel():]
         cells = torch.empty(n, dtype=torch.int32, device=rt.device) if want_cells else None
         stream = torch.cuda.current_stream(dev).cuda_stream
         _lib.check(lib.ocsc_apply_cells(h, rt.data_ptr(), n, qt.data_ptr(), n, nmesh, E, float(zstep), rm, scale,
@@ -154,7 +154,7 @@ def _kick(proc, p_array, zstep, want_cells):
         if direct:
             ctx.download(rt, host)
         else:
-            r[...] = rt.reshape(6, n).cpu().numpy()
+            r[...] = rt.reshape(host.shape).cpu().numpy()
     return cells.cpu().numpy() if cells is not None else None
 
 
