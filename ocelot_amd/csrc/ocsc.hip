@@ -888,25 +888,25 @@ bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // per thread up to 150k (20k / 31^3 FP64 128 us, 155 with eight, which leave
 // the chip idle; 100k / 31^3 136, 155; 160k / 31^3 150, 158) and eight above
 // (449k / 63^3 FP64 with two particles at 60 sigma 168, 210 with one; 4M /
-// 63^3 FP64 923, 952 with four).  In cell order two particles per thread in both
-// forms (us per step of a first call of 20, with two, four, eight: 50k / 31^3
-// mixed 95, 98, 101, FP64 97, 104, 108; 2M / 63^3 mixed 203, 207, 204, FP64 220,
-// 227, 225; 5M / 127^3 mixed 492, 494, 497; 10M / 127^3 mixed 722, 721, 728; the
-// most it loses is 1.5 per cent against eight, at 1M to 2M / 127^3 mixed, 354, 361,
-// 351).
-constexpr int64_t kDepOneMax = 150000;
-int dep_tile(const ocsc_ctx* c, int64_t n, bool ordered) {
+// 63^3 FP64 923, 952 with four).  In cell order two particles per thread where
+// workgroups are few or cells hold many (us per step of a first call of 20, with
+// two, eight: 50k / 31^3 mixed 95, 101, FP64 97, 108; 2M / 63^3 mixed 203, 204,
+// FP64 220, 225; 5M / 63^3 FP64 374, 390), eight where a table of two per thread
+// finds each cell a few times only (1M / 127^3 mixed 313, 307, FP64 374, 357; 2M /
+// 127^3 FP64 421, 415; 10M / 127^3 mixed 777, 756, from graphs 800, 770).
+constexpr int64_t kDepOneMax = 150000, kDepWideMin = 400000, kDepWideDensity = 6;
+int dep_tile(const ocsc_ctx* c, int64_t n, int64_t ncell, bool ordered) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return 6;
+  if (ordered) return n >= kDepWideMin && n < kDepWideDensity * ncell ? 0 : 6;
   return n <= kDepOneMax ? 5 : 0;
 }
 
 // the deposit variant the context's options select
 template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
-                    int32_t* cells, int64_t n, bool ordered, hipStream_t st) {
+                    int32_t* cells, int64_t n, int64_t ncell, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = dep_tile(c, n, ordered);
+  const int t = dep_tile(c, n, ncell, ordered);
   if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
   if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \
@@ -1086,7 +1086,7 @@ int enqueue_kick(ocsc_ctx* c, Lane& L, const Geometry& g, double* r, int64_t ld,
   } else if (o.bins) {
     launch_bin_deposit<NWORD>(R, q, L.sc, (unsigned long long*)L.grid.p, g, n, *o.bins, st);
   } else {
-    launch_deposit<NWORD>(c, R, q, L.sc, (unsigned long long*)L.grid.p, o.cells, n, o.ordered || sb, st);
+    launch_deposit<NWORD>(c, R, q, L.sc, (unsigned long long*)L.grid.p, o.cells, n, g.ncell, o.ordered || sb, st);
   }
   LAUNCHCHK("deposit");
   mark(3);

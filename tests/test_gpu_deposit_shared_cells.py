@@ -54,16 +54,19 @@ def test_shared_cells_give_the_bits_of_the_plain_atomics(n, mesh, far, prec):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
-@pytest.mark.parametrize("n", [511, 513, 1_000_001])
-def test_cell_order_with_the_kicks_clear(n, prec):
+@pytest.mark.parametrize("n,mesh", [(511, (17, 19, 15)), (513, (17, 19, 15)), (1_000_001, (17, 19, 15)),
+                                    (399_999, (47, 31, 63)), (400_000, (47, 31, 63)), (550_745, (47, 31, 63)),
+                                    (550_746, (47, 31, 63))])
+def test_cell_order_with_the_kicks_clear(n, mesh, prec):
     """Tracking steps after the first deposit into the grid that the mixed form's
-    kick has cleared: the same bits with every tile, and with pass B's clear."""
+    kick has cleared: the same bits with every tile (on both sides of the rule's
+    lines: 400000 particles, six per cell), and with pass B's clear."""
     from ocelot_amd import SpaceCharge, track_drift
     out = []
     for opts in (dict(), dict(deposit_tile=2), dict(deposit_tile=3), dict(grid_clear=0)):
         d = _bunch(n, 0)
         with _options(**opts):
-            track_drift(d, SpaceCharge(nmesh_xyz=[17, 19, 15], precision=prec), L=0.1, dz=0.1, nsteps=4)
+            track_drift(d, SpaceCharge(nmesh_xyz=list(mesh), precision=prec), L=0.1, dz=0.1, nsteps=4)
         out.append(d.rparticles.clone())
     assert all(torch.equal(out[0], o) for o in out[1:])
 
