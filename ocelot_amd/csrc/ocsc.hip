@@ -888,16 +888,18 @@ bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // per thread up to 150k (20k / 31^3 FP64 128 us, 155 with eight, which leave
 // the chip idle; 100k / 31^3 136, 155; 160k / 31^3 150, 158) and eight above
 // (449k / 63^3 FP64 with two particles at 60 sigma 168, 210 with one; 4M /
-// 63^3 FP64 923, 952 with four).  In cell order two particles per thread where
-// workgroups are few or cells hold many (us per step of a first call of 20, with
-// two, eight: 50k / 31^3 mixed 95, 101, FP64 97, 108; 2M / 63^3 mixed 203, 204,
-// FP64 220, 225; 5M / 63^3 FP64 374, 390), eight where a table of two per thread
-// finds each cell a few times only (1M / 127^3 mixed 313, 307, FP64 374, 357; 2M /
-// 127^3 FP64 421, 415; 10M / 127^3 mixed 777, 756, from graphs 800, 770).
-constexpr int64_t kDepOneMax = 150000, kDepWideMin = 400000, kDepWideDensity = 6;
-int dep_tile(const ocsc_ctx* c, int64_t n, int64_t ncell, bool ordered) {
+// 63^3 FP64 923, 952 with four).  In cell order two particles per thread (us per
+// tracking step with two, eight: 50k / 31^3 mixed 95, 101, FP64 97, 108; 400k /
+// 63^3 FP64 from graphs 139, 152; 800k / 63x63x95 FP64 with LSC and moments 314,
+// 331; 2M / 63^3 mixed 203, 204, FP64 220, 225; 5M / 63^3 FP64 374, 390), but eight
+// in the mixed form where a table of two per thread meets each cell a few times
+// only (flat-top bunches: 1M / 127^3 313, 307; 2M / 127^3 368, 362; 10M / 127^3 777,
+// 756, from graphs 800, 770).  The FP64 form gains there when launched one by one
+// (1M / 127^3 374, 357) and loses from graphs (800k / 127^3 341, 348): two.
+constexpr int64_t kDepOneMax = 150000, kDepWideMin = 1000000, kDepWideDensity = 6;
+int dep_tile(const ocsc_ctx* c, int64_t n, int64_t ncell, bool ordered, int nword) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return n >= kDepWideMin && n < kDepWideDensity * ncell ? 0 : 6;
+  if (ordered) return nword == 1 && n >= kDepWideMin && n < kDepWideDensity * ncell ? 0 : 6;
   return n <= kDepOneMax ? 5 : 0;
 }
 
@@ -906,7 +908,7 @@ template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
                     int32_t* cells, int64_t n, int64_t ncell, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = dep_tile(c, n, ncell, ordered);
+  const int t = dep_tile(c, n, ncell, ordered, NWORD);
   if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
   if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \
