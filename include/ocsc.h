@@ -350,9 +350,8 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * deposit and the kick (1, default) or gathers them into a cell-ordered
  * copy of the rows first (0); bit-identical results.  "deposit_tile": particles per thread and
  * LDS hash slots of the deposit, 0 (default) by the rows' order and number (in
- * cell order 2 and 512, FP64 256, or in the mixed form 8 and 2048 from 1000000
- * particles with fewer than six per cell; in the caller's order 1 and 256 up to
- * 150000 particles, above and in batches 8 and 2048, FP64 1024), 1 4 and 1024
+ * cell order 2 and 512, FP64 256, or 8 and 2048, FP64 1024, from 2500000
+ * particles on 1250000 cells; in the caller's order 1 and 256 up to 150000 particles, above and in batches 8 and 2048, FP64 1024), 1 4 and 1024
  * (FP64: 512), 2 16 and 4096 (FP64: 2048), 3 no table (one global atomic per
  * particle), 4 as in batches, with all of a thread's particle loads issued first; bit-identical results.  "batch_sort": see
  * ocsc_apply_batched.  "fft_plan": the transform plan, 0 LDS Stockham

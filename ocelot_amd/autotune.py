@@ -15,8 +15,8 @@ Knobs (``ocsc_set_option``):
 * ``deposit_agg``: runs of equal cells summed across the wavefront before
   the deposit's LDS table;
 * ``deposit_tile``: particles per thread and LDS hash slots of the deposit
-  (0: 2 x 512 (FP64 256), or in the mixed form 8 x 2048 by the number of
-  particles and cells; 1: 4 x 1024 (512), 2: 16 x 4096 (2048), 4: 8 x 2048 (1024) with every
+  (0: 2 x 512 (FP64 256) or 8 x 2048 (1024), by the number of particles and
+  cells; 1: 4 x 1024 (512), 2: 16 x 4096 (2048), 4: 8 x 2048 (1024) with every
   particle's loads issued first);
 * ``permute_rec``: permutations of the tracking copy through 64-byte
   particle records or row by row;

@@ -889,17 +889,19 @@ bool bin_buffers(Lane& L, const Geometry& g, int nword, int64_t n, BinBufs* B) {
 // the chip idle; 100k / 31^3 136, 155; 160k / 31^3 150, 158) and eight above
 // (449k / 63^3 FP64 with two particles at 60 sigma 168, 210 with one; 4M /
 // 63^3 FP64 923, 952 with four).  In cell order two particles per thread (us per
-// tracking step with two, eight: 50k / 31^3 mixed 95, 101, FP64 97, 108; 400k /
-// 63^3 FP64 from graphs 139, 152; 800k / 63x63x95 FP64 with LSC and moments 314,
-// 331; 2M / 63^3 mixed 203, 204, FP64 220, 225; 5M / 63^3 FP64 374, 390), but eight
-// in the mixed form where a table of two per thread meets each cell a few times
-// only (flat-top bunches: 1M / 127^3 313, 307; 2M / 127^3 368, 362; 10M / 127^3 777,
-// 756, from graphs 800, 770).  The FP64 form gains there when launched one by one
-// (1M / 127^3 374, 357) and loses from graphs (800k / 127^3 341, 348): two.
-constexpr int64_t kDepOneMax = 150000, kDepWideMin = 1000000, kDepWideDensity = 6;
-int dep_tile(const ocsc_ctx* c, int64_t n, int64_t ncell, bool ordered, int nword) {
+// tracking step with two, eight: 50k / 31^3 mixed 95, 101, FP64 97, 108; 800k /
+// 63x63x95 FP64 with LSC and moments 314, 331; 2M / 95^3 FP64 from graphs 331, 347;
+// 5M / 63^3 FP64 374, 390; 10M / 95^3 FP64 771, 779; 50M / 95^3 mixed 2645, 2657),
+// but eight for many particles on large meshes, where a table of two per thread
+// meets each cell a few times only (flat-top bunches: 3M / 127^3 mixed from graphs
+// 425, 417; 3M / 159^3 FP64 1430, 1408; 10M / 111^3 mixed 719, 705; 10M / 127^3 mixed
+// 776, 761; 10M / 255^3 mixed 2506, 2425, FP64 3075, 2914; 50M / 255^3 FP64 6028,
+// 5810).  Near the lines the two are within 1.5% of each other, either way by the
+// bunch's shape (3M / 111^3 mixed 383, 381, Gaussian 365, 370).
+constexpr int64_t kDepOneMax = 150000, kDepWideMin = 2500000, kDepWideCells = 1250000;
+int dep_tile(const ocsc_ctx* c, int64_t n, int64_t ncell, bool ordered) {
   if (c->deposit_tile || c->deposit_xcd || c->deposit_agg) return c->deposit_tile;
-  if (ordered) return nword == 1 && n >= kDepWideMin && n < kDepWideDensity * ncell ? 0 : 6;
+  if (ordered) return n >= kDepWideMin && ncell >= kDepWideCells ? 0 : 6;
   return n <= kDepOneMax ? 5 : 0;
 }
 
@@ -908,7 +910,7 @@ template <int NWORD>
 void launch_deposit(const ocsc_ctx* c, Rows R, const double* q, KickScalars* sc, unsigned long long* grid,
                     int32_t* cells, int64_t n, int64_t ncell, bool ordered, hipStream_t st) {
   const int v = (c->deposit_xcd ? 4 : 0) + (c->deposit_agg ? 2 : 0);
-  const int t = dep_tile(c, n, ncell, ordered, NWORD);
+  const int t = dep_tile(c, n, ncell, ordered);
   if (t == 5) return launch_deposit_t<NWORD, false, false, 5>(R, q, sc, grid, cells, n, st);
   if (t == 6) return launch_deposit_t<NWORD, false, false, 6>(R, q, sc, grid, cells, n, st);
 #define OCSC_DEP(V, T)                                                                                 \

@@ -55,12 +55,12 @@ def test_shared_cells_give_the_bits_of_the_plain_atomics(n, mesh, far, prec):
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("n,mesh", [(511, (17, 19, 15)), (513, (17, 19, 15)), (1_000_001, (17, 19, 15)),
-                                    (999_999, (63, 63, 63)), (1_000_000, (63, 63, 63)), (1_500_281, (63, 63, 63)),
-                                    (1_500_282, (63, 63, 63))])
+                                    (2_499_999, (127, 103, 97)), (2_500_000, (127, 103, 97)),
+                                    (2_500_000, (127, 103, 95))])
 def test_cell_order_with_the_kicks_clear(n, mesh, prec):
     """Tracking steps after the first deposit into the grid that the mixed form's
     kick has cleared: the same bits with every tile (on both sides of the rule's
-    lines: a million particles, six per cell), and with pass B's clear."""
+    lines: 2500000 particles, 1250000 cells), and with pass B's clear."""
     from ocelot_amd import SpaceCharge, track_drift
     out = []
     for opts in (dict(), dict(deposit_tile=2), dict(deposit_tile=3), dict(grid_clear=0)):

@@ -1,6 +1,6 @@
 """The tiles the deposit takes by itself: one particle per thread for small
 bunches in the caller's order, eight above; in cell order two, or eight for
-many particles over more cells.  Cell sums are integers, so every tile gives the same
+many particles on large meshes.  Cell sums are integers, so every tile gives the same
 bits as the table of option deposit_tile = 1, on both sides of the rule's line
 and where a wavefront's lane pairs are half empty."""
 import numpy as np
