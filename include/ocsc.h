@@ -351,10 +351,11 @@ int ocsc_apply_batched(ocsc_ctx* ctx, const ocsc_bunch* bunches, int nb, int pre
  * copy of the rows first (0); bit-identical results.  "deposit_tile": particles per thread and
  * LDS hash slots of the deposit, 0 (default) by the rows' order and number (in
  * cell order 2 and 512, FP64 256, or 8 and 2048, FP64 1024, from 2500000
- * particles on 1250000 cells; in the caller's order 1 and 256 up to 150000 particles, above and in batches 8 and 2048, FP64 1024), 1 4 and 1024
- * (FP64: 512), 2 16 and 4096 (FP64: 2048), 3 no table (one global atomic per
- * particle), 4 as in batches, with all of a thread's particle loads issued first; bit-identical results.  "batch_sort": see
- * ocsc_apply_batched.  "fft_plan": the transform plan, 0 LDS Stockham
+ * particles on 1250000 cells; in the caller's order 1 and 256 up to 150000
+ * particles, above and in batches 8 and 2048, FP64 1024), 1 4 and 1024 (FP64:
+ * 512), 2 16 and 4096 (FP64: 2048), 3 no table (one global atomic per
+ * particle), 4 as in batches, with all of a thread's particle loads issued
+ * first; bit-identical results.  "batch_sort": see ocsc_apply_batched.  "fft_plan": the transform plan, 0 LDS Stockham
  * passes, radix 16 where every thread gets a butterfly (else 8), 1 radix 8
  * in every pass, 2 half as many columns per workgroup, 3 the two field
  * passes with 256 threads per workgroup (radix 16 throughout) (1 to 3: mixed
