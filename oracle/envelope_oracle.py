@@ -1,6 +1,6 @@
 """FP64 CPU oracle for the beam moments of Ocelot's get_envelope.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker for ``ocsc_moments`` /
+TEST INFRASTRUCTURE ONLY.  This module is the oracle for ``ocsc_moments`` /
 ``ocelot_amd.get_envelope``: a numpy restatement of
 ocelot/cpbd/beam/analysis.py:27-224 (bounds with slice=None, dispersion from
 tws_i or estimated with auto_disp, the px/py correction factor, the twelve

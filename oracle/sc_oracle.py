@@ -1,6 +1,6 @@
 """FP64 CPU oracle for Ocelot's 3D space-charge kick.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker: it restates, in numpy and
+TEST INFRASTRUCTURE ONLY.  This module is the oracle: it restates, in numpy and
 scipy, the algorithm of ``SpaceCharge.apply`` from the reference
 (ocelot/cpbd/sc.py:76-251) and of the two coordinate maps it uses
 (ocelot/cpbd/coord_transform.py:16-96).  Only ``tests/``,

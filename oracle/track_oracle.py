@@ -1,6 +1,6 @@
 """FP64 CPU oracle for the tracking loop on a drift line with space charge.
 
-TEST INFRASTRUCTURE ONLY.  This module is the checker for
+TEST INFRASTRUCTURE ONLY.  This module is the oracle for
 ``ocelot_amd.track_drift``: it restates the loop of the reference's
 ``track()`` (ocelot/cpbd/track.py:462-485) on a line of drifts and markers,
 with the navigator's split of each step into element sections
